@@ -252,8 +252,69 @@ static bool ring_preferred(int64_t M, int epi, bool pro, int64_t N, int64_t K, i
          ring_tiles(epi, (int)N, 16) >= (int64_t)kRingTailMinTiles * cus;
 }
 
+// FLOW: every projection with a prologue, SwiGLU and argmax whose x rows fit its registers.
+static bool flow_fits(int64_t M, int epi, bool pro, int64_t K) {
+  return K % 8 == 0 && K <= INT32_MAX && flow_segments((int)K) <= kFlowMaxSegments && M <= kFlowMaxRows &&
+         flow_supported((int)M, (int)K, 16, epi, pro);
+}
+
+// The MFMA kind's LDS-fed form: the fewest rows per tile that give every tile a CU of its own
+// (x is read once per tile, so taller tiles read it less; more tiles than CUs run a second, partial
+// round). With the residual add, us per graph node on MI355X at M = 8 / 24, that choice against
+// 16-row tiles: 2048 x 6144 (8 rows) 6.9 / 9.7 against 8.5 / 11.2, 2560 x 9728 (12 rows)
+// 11.6 / 15.8 against 12.6 / 16.9, 5120 x 15360 (20 rows) 27.0 / 33.0 against 36.7 / 49.4,
+// 6144 x 4096 (24 rows) 10.7 / 12.3 against 13.0 / 16.2. 24-row tiles of 25..32 x rows fit the LDS
+// with four waves only. Past 24 rows per CU two smaller workgroups share a CU: 16 rows
+// (8192 x 4096, M = 8: 14.3 against 16.5 with 32), 32 from 17 x rows (M = 32: 17.9 against 18.3).
+struct MfmaLdsDefault {
+  int rows, kw;
+};
+static MfmaLdsDefault mfma_lds_default(int64_t M, int epi, bool pro, int64_t N, int64_t K, int cus) {
+  auto fits = [&](int rows, int kw) { return mfma_lds_supported((int)M, (int)K, rows, kw, epi, pro); };
+  if (K > INT32_MAX) return {0, 0};
+  if (epi == FTK_EPI_STORE) {
+    for (int rows = 8; rows <= 24; rows += 4)
+      if ((N + rows - 1) / rows <= cus)
+        for (int kw : {8, 4})
+          if (fits(rows, kw)) return {rows, kw};
+    if (M > 16 && fits(32, 4)) return {32, 4};
+  }
+  if (epi == FTK_EPI_ARGMAX && fits(16, 8)) return {16, 8};
+  // (A norm's gain beside the rings: long rows leave room for the smaller workgroups only, or none.)
+  const int rows = epi == FTK_EPI_SWIGLU ? 32 : 16;
+  return fits(rows, 4) ? MfmaLdsDefault{rows, 4} : MfmaLdsDefault{0, 0};
+}
+
 constexpr int kMfmaDefaultUnroll = 4;
 constexpr int kMfmaDefaultWaves = 16;
+
+// Where FLOW (a prologue, SwiGLU or argmax) or the MFMA kind's LDS-fed form (a plain STORE) comes
+// before QUAD, STAGE, STREAM and GEMV. us per graph node on MI355X over distinct weights, the kind
+// there otherwise against the one chosen here:
+//   5..16 rows, K without a RING build: norm 4096 x 1024 at M = 8 / 16 QUAD 5.6 / MFMA's registers
+//     7.0 against 5.3 / 5.3; gate/up 6144 x 1024 7.5 / 8.5 against 5.8 / 6.3, 19456 x 2560 30 / 35
+//     against 20 / 19; lm_head 151936 x 1024 184 / 228 against 55 / 55.
+//   2..4 rows: where only GEMV is built (norm 4096 x 2560 at M = 2 / 4 8.2 / 10.8 against 8.3 / 8.4,
+//     gate/up 19456 x 2560 23 / 34 against 20 / 20), lm_head (50257 x 2048 43.8 / 44.6 against 38.4),
+//     and at 3..4 rows gate/up (6144 x 1024 6.0 against 5.8, 12288 x 2048 12.0 against 11.4) and plain
+//     projections of fewer than 16 rows per CU (2048 x 2048 5.0 against 4.2, 1536 x 4096 6.1
+//     against 4.9). Wider plain ones keep the STREAM launches of the 8B shapes.
+//   one row, where only GEMV is built: plain projections (1920 x 5760 9.9 against 6.0, 2560 x 9728 17.6
+//     against 10.7, 5120 x 15360 29.6 against 27.7; K in whole 128-byte lines, as GEMV's loads have no
+//     such need), and FLOW from 8192 outputs (gate/up 19456 x 2560 23.8 against 20.4; norm
+//     4096 x 2560 7.4 against 8.4).
+//   17..32 rows: everything (callers that want the native GEMM there do not come here).
+static bool wide_first(int64_t M, int epi, bool pro, int64_t N, int64_t K, int cus, bool quad, bool stage, bool stream) {
+  const bool plain = !pro && epi == FTK_EPI_STORE;
+  if (!plain && !flow_fits(M, epi, pro, K)) return false;
+  if (M > 4) return !stage && !(M <= 8 && quad && K == 4096);
+  if (M > 1) {
+    if (plain) return !stream || (M >= 3 && N <= 12ll * cus);
+    return !(quad || stream) || (K != 4096 && (epi == FTK_EPI_ARGMAX || (M >= 3 && epi == FTK_EPI_SWIGLU)));
+  }
+  if (stream) return false;
+  return plain ? K % 64 == 0 : gemv_outputs(epi, (int)N) >= 8192;
+}
 
 static int64_t argmax_keys_bytes(int grid, int64_t M) { return kWsKeys + (int64_t)grid * M * 8; }
 
@@ -285,15 +346,23 @@ static int plan(int64_t M, int64_t N, int64_t K, int epi, int cus, const ftk_con
     // 768 x 4096 with the norm, at M = 5: 64 RING tiles 7.80 us, QUAD 6.55).
     const bool ring = rd.kw != 0 && (ring_tiles(epi, (int)N, rd.rows) >= cus / 2 || !quad ||
                                      !quad_preferred(M, epi, pro));
+    // The kinds whose x slice or ring is built for a few K (STREAM, QUAD, STAGE, RING) where they
+    // are the fastest; for any other K, FLOW and the MFMA kind's LDS-fed form (wide_first).
+    const bool stream = M <= 4 && stream_default(M, epi, N, K).rpw != 0;
     if (K % 8)
       kind = FTK_KIND_GENERIC;
     else if (ring)
       kind = FTK_KIND_RING;
+    else if (ring_ok && wide_first(M, epi, pro, N, K, cus, quad && quad_preferred(M, epi, pro), stage, stream))
+      // (SwiGLU and argmax without the norm from 17 rows: the tile form unless a caller asks for FLOW.)
+      kind = (!pro && (epi == FTK_EPI_STORE || M > 16)) || !flow_fits(M, epi, pro, K)
+                 ? FTK_KIND_MFMA
+                 : FTK_KIND_FLOW;
     else if (quad && quad_preferred(M, epi, pro))
       kind = FTK_KIND_QUAD;
     else if (stage)
       kind = FTK_KIND_STAGE;
-    else if (M <= 4 && stream_default(M, epi, N, K).rpw)
+    else if (stream)
       kind = FTK_KIND_STREAM;
     else if (M <= 4)
       kind = FTK_KIND_GEMV;
@@ -446,6 +515,24 @@ static int plan(int64_t M, int64_t N, int64_t K, int epi, int cus, const ftk_con
       p->workspace_bytes = kWsClaim + 4;
     return FTK_OK;
   }
+  if (kind == FTK_KIND_FLOW) {
+    const int waves = cfg && cfg->waves ? cfg->waves : kFlowWaves;
+    const int rows = cfg && cfg->rows_per_wave ? cfg->rows_per_wave : 16;
+    if (M > kFlowMaxRows || flow_segments((int)K) > kFlowMaxSegments) return FTK_ERR_UNSUPPORTED;
+    if (waves != kFlowWaves || !flow_supported((int)M, (int)K, rows, epi, pro)) return FTK_ERR_INVALID;
+    p->rows_per_wave = rows;
+    p->unroll = flow_depth(rows);
+    p->waves = waves;
+    p->threads = 64 * waves;
+    p->tiles = flow_tiles(epi, (int)N, rows);
+    // One workgroup per CU (its LDS fills the CU), in a grid of full XCD runs (ring_tile).
+    const int64_t units = (int64_t)(cfg && cfg->groups_per_cu ? cfg->groups_per_cu : 1) * cus;
+    p->grid = persistent_programs(p->tiles, (int)(units < p->tiles ? units : p->tiles));
+    const int even = (p->grid + 7) / 8 * 8;
+    if (even <= p->tiles) p->grid = even;
+    p->workspace_bytes = epi == FTK_EPI_ARGMAX ? argmax_keys_bytes(p->grid, M) : 0;
+    return FTK_OK;
+  }
   if (kind == FTK_KIND_MFMA_STREAM) {
     if (M > kMstreamMaxRows) return FTK_ERR_UNSUPPORTED;
     const MstreamDefault d = mstream_default(M, epi, pro, N, K);
@@ -469,7 +556,23 @@ static int plan(int64_t M, int64_t N, int64_t K, int epi, int cus, const ftk_con
     return FTK_OK;
   }
   if (kind == FTK_KIND_MFMA) {
-    // Defaults from the MI355X sweep: 16 rows (SwiGLU: one gate + one up subtile)
+    // The LDS-fed form: unroll 1, or no launch fields at all. It takes no residual add in its prologue.
+    const bool given = cfg && (cfg->rows_per_wave || cfg->unroll || cfg->waves);
+    const MfmaLdsDefault d = mfma_lds_default(M, epi, pro, N, K, cus);
+    if (ring_ok && (given ? cfg->unroll == 1 : d.rows != 0)) {
+      const int rows = given && cfg->rows_per_wave ? cfg->rows_per_wave : d.rows;
+      const int waves = given && cfg->waves ? cfg->waves : d.kw;
+      if (!mfma_lds_supported((int)M, (int)K, rows, waves, epi, pro)) return FTK_ERR_INVALID;
+      p->rows_per_wave = rows;
+      p->unroll = 1;
+      p->waves = waves;
+      p->threads = 64 * waves;
+      p->tiles = flow_tiles(epi, (int)N, rows);
+      p->grid = p->tiles;
+      p->workspace_bytes = epi == FTK_EPI_ARGMAX ? argmax_keys_bytes(p->grid, M) : 0;
+      return FTK_OK;
+    }
+    // Explicit launches from the MI355X sweep: 16 rows (SwiGLU: one gate + one up subtile)
     // per workgroup of 16 waves; 32 rows once M > 16 (two MFMA column blocks).
     const int rows = cfg && cfg->rows_per_wave ? cfg->rows_per_wave : (epi == FTK_EPI_SWIGLU || M > 16 ? 32 : 16);
     if (rows % 16) return FTK_ERR_INVALID;
@@ -492,7 +595,7 @@ static int plan(int64_t M, int64_t N, int64_t K, int epi, int cus, const ftk_con
 // Workspace a call needs: argmax keys, and the RMSNorm row scales of the MFMA kind.
 static int64_t call_workspace(const ftk_plan& p, int epi, bool pro) {
   if (epi == FTK_EPI_ARGMAX) return p.workspace_bytes;
-  if (p.kind == FTK_KIND_MFMA && pro) return kWsKeys;
+  if (p.kind == FTK_KIND_MFMA && pro && p.unroll != 1) return kWsKeys;
   return 0;
 }
 
@@ -629,6 +732,24 @@ int64_t ftk_project_workspace_bytes(int64_t M, int64_t N, int64_t K, int epilogu
   return p.workspace_bytes;
 }
 
+// Tiles of RT rows taken as the FLOW kernels take them (with one tile per workgroup: tile b).
+static void flow_coverage(int rt, int grid, int tiles, int epilogue, int N, int32_t* counts, int64_t outputs,
+                          int64_t* max_row) {
+  const int per = flow_out_per_tile(epilogue, rt);
+  for (int b = 0; b < grid; ++b)
+    for (int i = 0; b + i * grid < tiles; ++i) {
+      const int tile = grid == tiles ? b : ring_tile(b, i, grid, tiles);
+      for (int r = 0; r < rt; ++r) {
+        const int64_t row = flow_weight_row(epilogue, tile, r, N, rt);
+        if (row > *max_row) *max_row = row;
+      }
+      for (int r = 0; r < per; ++r) {
+        const int64_t col = (int64_t)tile * per + r;
+        if (col < outputs) counts[col] += 1;
+      }
+    }
+}
+
 int ftk_plan_coverage(const ftk_plan* p, int64_t N, int epilogue, int32_t* counts, int64_t outputs,
                       int64_t* max_row) {
   if (p == nullptr || counts == nullptr || max_row == nullptr) return FTK_ERR_INVALID;
@@ -647,9 +768,14 @@ int ftk_plan_coverage(const ftk_plan* p, int64_t N, int epilogue, int32_t* count
     return FTK_OK;
   }
   if (p->kind == FTK_KIND_MFMA) {
-    // Workgroup b owns tile b: T subtiles of 16 weight rows over all of K.
+    // Workgroup b owns tile b: T subtiles of 16 weight rows (the LDS-fed form: RT rows) over all of K.
+    if (p->grid != p->tiles) return FTK_ERR_INVALID;
+    if (p->unroll == 1) {
+      flow_coverage(p->rows_per_wave, p->grid, p->tiles, epilogue, (int)N, counts, outputs, max_row);
+      return FTK_OK;
+    }
     const int t = p->rows_per_wave / 16;
-    if (t < 1 || p->grid != p->tiles) return FTK_ERR_INVALID;
+    if (t < 1) return FTK_ERR_INVALID;
     const int per = mfma_out_per_tile(epilogue, t);
     for (int b = 0; b < p->grid; ++b) {
       for (int sub = 0; sub < t; ++sub)
@@ -683,6 +809,11 @@ int ftk_plan_coverage(const ftk_plan* p, int64_t N, int epilogue, int32_t* count
           if (col < outputs) counts[col] += 1;
         }
       }
+    return FTK_OK;
+  }
+  if (p->kind == FTK_KIND_FLOW) {
+    if (p->grid < 1 || p->grid > p->tiles) return FTK_ERR_INVALID;
+    flow_coverage(p->rows_per_wave, p->grid, p->tiles, epilogue, (int)N, counts, outputs, max_row);
     return FTK_OK;
   }
   if (p->kind == FTK_KIND_RING) {
@@ -818,11 +949,14 @@ static int project_impl(const void* x, const ftk_rows* rows, const void* gamma, 
   a.x_ids_bytes = r.x_ids_bytes;
   a.x_rows = r.x_rows;
   a.out_add = (const uint16_t*)out_add;
-  // The MFMA kind's projection reads the pre-pass's stored rows: it needs sum.
-  if (p.kind == FTK_KIND_MFMA && (r.residual != nullptr || r.x_ids != nullptr) && r.sum == nullptr)
+  // The MFMA kind's LDS-fed form loads x rows as they are: a residual add takes the explicit
+  // form's pre-pass, whose stored rows the projection then reads (it needs sum).
+  const bool lds_form = p.kind == FTK_KIND_MFMA && p.unroll == 1;
+  if (p.kind == FTK_KIND_MFMA && !lds_form && (r.residual != nullptr || r.x_ids != nullptr) && r.sum == nullptr)
     return FTK_ERR_UNSUPPORTED;
   // The RING kind loads x rows as they are: no residual add in its prologue.
   if (p.kind == FTK_KIND_RING && r.residual != nullptr) return FTK_ERR_UNSUPPORTED;
+  if (p.kind == FTK_KIND_FLOW && (r.residual != nullptr || out_add != nullptr)) return FTK_ERR_UNSUPPORTED;
   // Row sums of squares travel between RING launches only (16-row STORE tiles write them).
   if (r.sumsq != nullptr && p.kind != FTK_KIND_RING) return FTK_ERR_UNSUPPORTED;
   if (r.sumsq_out != nullptr && (p.kind != FTK_KIND_RING || p.rows_per_wave != 16)) return FTK_ERR_UNSUPPORTED;
@@ -856,9 +990,15 @@ static int project_impl(const void* x, const ftk_rows* rows, const void* gamma, 
   } else if (p.kind == FTK_KIND_RING) {
     RingShape g = {p.unroll, p.waves, p.grid, p.tiles, p.rows_per_wave};
     e = launch_ring(a, epilogue, g, s);
+  } else if (p.kind == FTK_KIND_FLOW) {
+    FlowShape g = {p.rows_per_wave, p.grid, p.tiles};
+    e = launch_flow(a, epilogue, g, s);
   } else if (p.kind == FTK_KIND_GEMV) {
     GemvShape g = {p.rows_per_wave, p.unroll, p.waves, p.grid, p.tiles, (size_t)p.lds_bytes};
     e = launch_gemv(a, epilogue, g, s);
+  } else if (lds_form) {
+    MfmaLdsShape g = {p.rows_per_wave, p.waves, p.grid};
+    e = launch_mfma_lds(a, epilogue, g, s);
   } else {
     MfmaShape shape = {p.rows_per_wave / 16, p.unroll, p.waves, p.grid};
     MfmaArgs m;
@@ -961,7 +1101,9 @@ int ftk_lm_head_argmax_static_bf16(const void* x, const void* gamma, float eps, 
   if (st != FTK_OK) return st;
   // Every key slot the finalize pass reads is written earlier in the same call,
   // so the array needs no clearing between calls.
-  if (call_workspace(p, FTK_EPI_ARGMAX, gamma != nullptr) > FTK_STATIC_SCRATCH_BYTES) return FTK_ERR_TOO_LARGE;
+  // From 17 rows the bound is one key per row and 16-row tile, whatever the launch needs.
+  const int64_t keys = M > 16 ? argmax_keys_bytes((int)((V + 15) / 16), M) : call_workspace(p, FTK_EPI_ARGMAX, gamma != nullptr);
+  if (keys > FTK_STATIC_SCRATCH_BYTES) return FTK_ERR_TOO_LARGE;
   void* ws = nullptr;
   const int got = static_scratch(&ws);
   if (got != FTK_OK) return got;

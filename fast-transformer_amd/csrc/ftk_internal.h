@@ -60,6 +60,46 @@ __device__ __forceinline__ uint32_t store_bits(const ProjArgs& a, float s, int m
   return f32_to_bf16(bf16_to_f32(b) + bf16_to_f32(a.out_add[(size_t)m * a.N + n]));
 }
 
+// Four residual elements [m, n0 .. n0 + 3] of the STORE epilogue's add (zeros without one), loaded
+// together: whole and aligned rows in one 8-byte load, else four loads with the columns past N
+// re-reading the last one. A kernel issues this ahead of its last wait; loading each element where
+// it is added (store_bits) costs one memory round trip per element.
+__device__ __forceinline__ u32x2_t out_add4(const ProjArgs& a, int m, int n0) {
+  u32x2_t v = {0u, 0u};
+  if (a.out_add == nullptr) return v;
+  const uint16_t* r = a.out_add + (size_t)m * a.N;
+  if ((a.N & 3) == 0 && (reinterpret_cast<uintptr_t>(a.out_add) & 7) == 0) {
+    v = *reinterpret_cast<const u32x2_t*>(r + min(n0, a.N - 4));
+  } else {
+    const uint32_t e0 = r[min(n0, a.N - 1)], e1 = r[min(n0 + 1, a.N - 1)];
+    const uint32_t e2 = r[min(n0 + 2, a.N - 1)], e3 = r[min(n0 + 3, a.N - 1)];
+    v = u32x2_t{e0 | (e1 << 16), e2 | (e3 << 16)};
+  }
+  return v;
+}
+
+// store_bits of four outputs whose residual elements were loaded by out_add4.
+__device__ __forceinline__ void store_bits4(const ProjArgs& a, const f32x4_t& s, u32x2_t add, uint32_t (&bits)[4]) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r) bits[r] = f32_to_bf16(s[r]);
+  if (a.out_add == nullptr) return;
+  const uint32_t e[2] = {add[0], add[1]};
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    bits[r] = f32_to_bf16(bf16_to_f32(bits[r]) + ((r & 1) ? hi_f32(e[r >> 1]) : lo_f32(e[r >> 1])));
+}
+
+// Four BF16 outputs at columns n .. n + 3 of a row of `cols`: one 8-byte store where whole and aligned.
+__device__ __forceinline__ void store_row4(uint16_t* row, int n, int cols, const uint32_t (&bits)[4]) {
+  if (n + 3 < cols && (reinterpret_cast<uintptr_t>(row + n) & 7) == 0) {
+    *reinterpret_cast<u32x2_t*>(row + n) = u32x2_t{bits[0] | (bits[1] << 16), bits[2] | (bits[3] << 16)};
+  } else {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (n + r < cols) row[n + r] = (uint16_t)bits[r];
+  }
+}
+
 // ---- greedy argmax in one launch ------------------------------------------------
 // With a.fused, every tile workgroup publishes its best key per row, keys[wg M + m],
 // as an agent-scope store (coherent across the XCDs' L2s) of a non-zero word, and
@@ -294,6 +334,24 @@ struct MfmaArgs {
 };
 bool mfma_supported(int M, int t, int unroll, int waves, int epi);
 hipError_t launch_mfma(const ProjArgs& a, int epi, const MfmaShape& shape, const MfmaArgs& p, hipStream_t stream);
+
+// Launch shape of the FLOW kind.
+struct FlowShape {
+  int rows;      // RT: weight rows per tile (8, 12 or 16)
+  int grid;      // workgroups; workgroup wg takes tile ring_tile(wg, i, grid, tiles) at step i
+  int tiles;
+};
+bool flow_supported(int M, int K, int rt, int epi, bool pro);
+hipError_t launch_flow(const ProjArgs& a, int epi, const FlowShape& shape, hipStream_t stream);
+
+// Launch shape of the MFMA kind's LDS-fed form (one workgroup per tile).
+struct MfmaLdsShape {
+  int rows;   // RT: weight rows per tile
+  int waves;  // KW: waves per workgroup, splitting K in 128-wide segments
+  int grid;   // workgroups (one per tile)
+};
+bool mfma_lds_supported(int M, int K, int rt, int kw, int epi, bool pro);
+hipError_t launch_mfma_lds(const ProjArgs& a, int epi, const MfmaLdsShape& shape, hipStream_t stream);
 
 // Arguments of one split-KV decode-attention launch (engine/kernels/decode_attention.py:31-149).
 // A group is one (row, KV head) pair: group = row * kv_heads + kv_head.

@@ -218,6 +218,74 @@ FTK_HD constexpr int ring_max_depth(int c, int kw, int d, int nx, bool pro, int 
   return depth > 8 ? 8 : depth;
 }
 
+// ---- M = 1..32 with any K % 8 == 0 up to 5120: the FLOW kind ------------------------
+// A persistent walk as RING's (tile ring_tile(wg, i, G, tiles) at step i), with the
+// K segments dealt to 8 waves (wave kw: kw, kw + 8, ...; the last may be short) and
+// the x rows of a wave's segments in registers throughout. A tile is RT = 8, 12 or 16
+// weight rows, for SwiGLU RT / 2 gate rows and the matching up rows.
+constexpr int kFlowMaxRows = 32;
+constexpr int kFlowWaves = 8;
+constexpr int kFlowMaxSegments = 5;  // per wave
+// Loads of 4 x rows per unit a kernel is built for.
+FTK_HD constexpr int flow_x_loads(int m) { return m <= 4 ? 1 : m <= 8 ? 2 : m <= 16 ? 4 : m <= 24 ? 6 : 8; }
+FTK_HD constexpr int flow_segments(int k) { return ((k + 127) / 128 + kFlowWaves - 1) / kFlowWaves; }
+FTK_HD constexpr int flow_out_per_tile(int epi, int rt) { return epi == EPI_SWIGLU ? rt / 2 : rt; }
+FTK_HD int flow_tiles(int epi, int n_rows, int rt) {
+  const int per = flow_out_per_tile(epi, rt);
+  return (gemv_outputs(epi, n_rows) + per - 1) / per;
+}
+// Weight row of unit row r (0..RT-1) in tile t, clamped in bounds.
+FTK_HD int flow_weight_row(int epi, int t, int r, int n_rows, int rt) {
+  if (epi == EPI_SWIGLU) {
+    const int half = n_rows / 2, per = rt / 2;
+    int c = t * per + (r < per ? r : r - per);
+    c = c < half ? c : half - 1;
+    return r < per ? c : half + c;
+  }
+  const int row = t * rt + r;
+  return row < n_rows ? row : n_rows - 1;
+}
+// Weight units in flight per wave, x units staged at once (in 16 KiB per wave), and the
+// 16-byte slots of a wave's LDS that hold one or the other.
+FTK_HD constexpr int flow_depth(int rt) { return rt == 16 ? 4 : rt == 12 ? 5 : 8; }
+FTK_HD constexpr int flow_x_batch(int nx, int cm) { return cm * nx <= 16 ? cm : 16 / nx; }
+FTK_HD constexpr int flow_wave_slots(int nx, int cm, int rt) {
+  return flow_depth(rt) * 16 * rt > flow_x_batch(nx, cm) * 64 * nx ? flow_depth(rt) * 16 * rt
+                                                                   : flow_x_batch(nx, cm) * 64 * nx;
+}
+// Tiles whose per-wave partials fit beside the rings, the gain and the row sums (at most 4).
+FTK_HD constexpr int flow_parked(int nx, int cm, int rt, bool pro) {
+  const int mb = (nx + 3) / 4;
+  const int fixed = (kFlowWaves * flow_wave_slots(nx, cm, rt) + 256 * mb - 64 * nx) * 16 +
+                    kFlowWaves * (pro ? cm * 256 : 0) + kFlowWaves * 64 * mb + kFlowWaves * 128 + 256;
+  const int fit = (160 * 1024 - fixed) / (kFlowWaves * 1024 * mb);
+  return fit > 4 ? 4 : fit;
+}
+
+// ---- The MFMA kind's LDS-fed form: FLOW's tiles, one per workgroup -----------------
+// Tiles of RT = 8, 12, 16, 20, 24 or 32 weight rows (SwiGLU: 32) over all of K, for any
+// K % 8 == 0; x streams beside the weights. Units (128-wide K segments) of weights and
+// of x in flight per wave:
+FTK_HD constexpr int mfma_lds_w_units(int rt, int kw) { return rt == 32 ? 1 : 2; }
+FTK_HD constexpr int mfma_lds_x_units(int rt, int kw, int mb) { return mb == 1 && rt <= 20 ? 2 : 1; }
+FTK_HD constexpr int mfma_lds_wave_slots(int nx, int rt, int kw) {
+  return mfma_lds_w_units(rt, kw) * 16 * rt + mfma_lds_x_units(rt, kw, (nx + 3) / 4) * 64 * nx;
+}
+// Slots past the rings that operand reads of the last wave's last units may touch.
+FTK_HD constexpr int mfma_lds_pad_slots(int nx, int rt, int kw) {
+  const int mb = (nx + 3) / 4, t = (rt + 15) / 16;
+  const int x = 256 * mb - 64 * nx;
+  const int w = (mfma_lds_w_units(rt, kw) - 1) * 16 * rt + 256 * t - mfma_lds_wave_slots(nx, rt, kw);
+  return x > w ? (x > 0 ? x : 0) : (w > 0 ? w : 0);
+}
+// LDS of a workgroup: the rings and their pad, the gain (K > 0), row scales and argmax keys.
+FTK_HD constexpr int mfma_lds_bytes(int nx, int rt, int kw, int k) {
+  return (kw * mfma_lds_wave_slots(nx, rt, kw) + mfma_lds_pad_slots(nx, rt, kw)) * 16 + (k + 127) / 128 * 256 + 1024;
+}
+FTK_HD constexpr bool mfma_lds_shape(int nx, int rt, int kw) {
+  return mfma_lds_bytes(nx, rt, kw, 0) <= 160 * 1024 && kw * mfma_lds_wave_slots(nx, rt, kw) >= kw * ((rt + 15) / 16) * ((nx + 3) / 4) * 64;
+}
+
 // ---- workspace layout of one projection call (bytes) -----------------------
 // The row scales are written by the prologue pass before they are read. The
 // argmax key words are zero between calls: a workspace is zeroed when it is

@@ -56,28 +56,12 @@
 #include <type_traits>
 
 #include "ftk_device.h"
+#include "ftk_dma.h"
 #include "ftk_internal.h"
 
 namespace ftk {
 
 namespace {
-
-typedef __attribute__((address_space(1))) const void global_void_t;
-typedef __attribute__((address_space(3))) void lds_void_t;
-
-// 16 bytes per lane from `src` into LDS at dst + 16 lane (dst is wave-uniform).
-// AUX 2: non-temporal (the weights, read once per call); 0: cached (x).
-template <int AUX>
-__device__ __forceinline__ void dma16(const void* src, void* dst) {
-  __builtin_amdgcn_global_load_lds((global_void_t*)src, (lds_void_t*)dst, 16, 0, AUX);
-}
-
-// Wait until at most N vector memory instructions of this wave are outstanding.
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
 
 __device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
@@ -160,14 +144,6 @@ __device__ __forceinline__ uint32_t claim_add(unsigned* p) {
   uint32_t old;
   asm volatile("global_atomic_add %0, %1, %2, off sc0" : "=v"(old) : "v"(p), "v"(1u) : "memory");
   return old;
-}
-
-// Workgroup barrier for LDS traffic only. __syncthreads() also waits for every
-// vector memory operation (vmcnt(0)), which would empty the ring mid-walk.
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
 }
 
 template <int I, int N, class F>

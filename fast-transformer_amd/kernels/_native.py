@@ -19,10 +19,12 @@ STATIC_SCRATCH_BYTES = 1 << 20  # FTK_STATIC_SCRATCH_BYTES
 EPI_STORE, EPI_SWIGLU, EPI_ARGMAX = range(3)
 PLAN_PROLOGUE = 0x100  # FTK_PLAN_PROLOGUE
 PLAN_RESIDUAL = 0x200  # FTK_PLAN_RESIDUAL
-KIND_AUTO, KIND_GEMV, KIND_MFMA, KIND_GENERIC, KIND_STREAM, KIND_MFMA_STREAM, KIND_QUAD, KIND_STAGE, KIND_RING = range(9)
+KIND_AUTO, KIND_GEMV, KIND_MFMA, KIND_GENERIC, KIND_STREAM, KIND_MFMA_STREAM, KIND_QUAD, KIND_STAGE, KIND_RING, \
+    KIND_FLOW = range(10)
 ATTN_AUTO, ATTN_ROWS, ATTN_QUAD = range(3)
 ROPE_PREFILL, ROPE_ROWS, ROPE_TABLE = 0x1, 0x2, 0x4
 MAX_ROWS = 32
+FLOW_MAX_K = 5120  # K a FLOW wave's x registers hold
 
 _c_void_p, _i64, _int, _float = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_float
 

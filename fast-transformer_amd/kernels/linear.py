@@ -10,11 +10,12 @@ one rounding to BF16 (linear.py:1-6). Under them:
   * M = 2..16: MFMA kinds (4x4x4 blocks fed straight from 4-row x 256-byte
     loads, or 16x16x32 tiles fed through LDS), as the C library's planner picks;
     ragged K or an unaligned pointer takes a generic kernel with scalar loads;
-  * M = 17..32: torch's native GEMM by default (hipBLASLt measured faster there),
-    the way the reference keeps cuBLAS unless a timed kind beats it; the fused
-    forms run their norm / epilogue kernels around it. An explicit config, or
-    the first-use timing of the candidates (on unless FTK_TUNE=0), still
-    launches these kernels at any M.
+  * M = 17..32: the same MFMA kinds with two column blocks where they measured
+    faster than torch's native GEMM (``default_choice``), else that GEMM
+    (hipBLASLt), the way the reference keeps cuBLAS unless a timed kind beats it,
+    with the norm / epilogue kernels around it. An explicit config, or the
+    first-use timing of the candidates (on unless FTK_TUNE=0), launches these
+    kernels at any M.
 
 ``split_ok`` is accepted for signature compatibility. The result is always a
 contiguous BF16 tensor, which the reference allows ("may be" a Split,
@@ -48,10 +49,10 @@ _VALIDATED = {}
 #: come from the same kind of timing, done once on MI355X.
 TUNE = os.environ.get("FTK_TUNE", "1") != "0"
 
-#: From this many rows the planner's default is torch's native GEMM (hipBLASLt), as the reference
-#: keeps cuBLAS unless a timed kind beats it (linear.py:455-475). Measured on MI355X at Qwen3-8B
-#: shapes: at 32 rows hipBLASLt is 1.6-2.7x faster than these kernels; at 16 and fewer rows these
-#: kernels are faster on every projection (1.09x for down at 16 rows, up to 2.1x for O).
+#: From this many rows torch's native GEMM (hipBLASLt) is a default at some shapes, as the reference
+#: keeps cuBLAS unless a timed kind beats it (linear.py:455-475): ``default_choice`` says which. The
+#: forms without a selection (a residual in the prologue, the embedding gather) compose there.
+#: At 16 and fewer rows these kernels are faster on every projection.
 NATIVE_FROM_ROWS = 17
 
 
@@ -59,6 +60,41 @@ def prefer_native(rows, config=None):
     """Whether a call with no explicit launch choice goes to the native GEMM (plus separate norm /
     epilogue kernels for the fused forms)."""
     return config is None and rows >= NATIVE_FROM_ROWS
+
+
+#: CUs of an MI355X: the LDS-fed tiles (at most 24 rows) of a projection of up to 24 x CUS outputs
+#: run as one round of workgroups.
+CUS = 256
+
+
+def default_choice(op, rows, n, k):
+    """The launch choice of a call that was not timed: "native", or None for this library's kernels.
+
+    Up to 16 rows these kernels. From 17 rows they are the faster ones too wherever a whole tile per
+    CU fits (``linear`` and ``norm`` to 6144 outputs) or the walk keeps the x rows in registers (FLOW,
+    K <= 5120), us on MI355X against the native form at 24 rows: norm 6144 x 4096 15.4 / 18.0, gate/up
+    24576 x 4096 38.5 / 53.3, 19456 x 2560 22.6 / 30.2, lm_head 151936 x 4096 201 / 274, O 4096 x 4096
+    9.7 / 13.4, down 4096 x 12288 23.1 / 25.4. Other shapes, and weights of less than 4 MB (which
+    callers were promised as torch's own result there), stay native.
+    """
+    if rows < NATIVE_FROM_ROWS:
+        return None
+    if rows > MAX_ROWS or k % 8 or n * k < 1 << 21:
+        return "native"
+    if op in ("linear", "norm") and n <= 24 * CUS:
+        return None
+    return None if k <= _native.FLOW_MAX_K and op != "linear" else "native"
+
+
+def norm_apart(rows, k):
+    """Whether a norm + projection of this size runs as two launches by default: from 17 rows every
+    CU's normalisation of all x rows takes longer than the norm's own launch, unless rows are short
+    (24 rows: 6144 x 4096 17.7 us fused, 2.75 + 12.7 apart; 4096 x 1024 6.4 against 2.4 + 4.3)."""
+    return rows >= NATIVE_FROM_ROWS and k > 1024
+
+
+#: FLOW at its default shape: the walk for projections of more than one round of tiles.
+FLOW = _native.Config(_native.KIND_FLOW, 0, 0, 0, 0)
 
 
 def _fusable(flat, weight, norm_weight=None):
@@ -215,7 +251,11 @@ def rms_norm_linear(x, norm_weight, eps, weight, config=None, sumsq=None):
 
     def fused(cfg, w, inp=flat):
         y = torch.empty((inp.shape[0], w.shape[0]), device=inp.device, dtype=torch.bfloat16)
-        status = fused_project(inp, w, _native.EPI_STORE, y, norm_weight, eps, config=cfg, sumsq=sumsq)
+        if cfg is None and norm_apart(m, k):
+            walk = FLOW if w.shape[0] > 24 * CUS and k <= _native.FLOW_MAX_K else None
+            status = fused_project(rms_norm(inp, norm_weight, eps), w, _native.EPI_STORE, y, config=walk)
+        else:
+            status = fused_project(inp, w, _native.EPI_STORE, y, norm_weight, eps, config=cfg, sumsq=sumsq)
         return y if status == _native.FTK_OK else None
 
     if config is None and _fusable(flat, weight, norm_weight):
@@ -355,6 +395,9 @@ def _candidates(m, n, k, epilogue=_native.EPI_STORE, prologue=False):
         for rows in (16, 32):
             for kw, unroll in ((8, 4), (8, 8), (16, 4)):
                 configs.append((_native.KIND_MFMA_STREAM, rows, unroll, 1, kw))
+    configs.append((_native.KIND_FLOW, 16, 0, 1, 8))
+    for rows, waves in ((8, 8), (12, 8), (16, 8), (20, 8), (24, 8), (16, 4), (24, 4), (32, 4)):
+        configs.append((_native.KIND_MFMA, rows, 1, 0, waves))
     for rows, unroll, waves in ((16, 4, 4), (16, 8, 8), (32, 4, 8), (64, 2, 4)):
         configs.append((_native.KIND_MFMA, rows, unroll, 0, waves))
     p = _native.Plan()
@@ -464,7 +507,7 @@ def _inherit(op, x, weight, run, native, compare=None):
     m, k = x.shape
     n = weight.shape[0]
     key = _key(op, x.device, m, n, k)
-    default = "native" if prefer_native(m) else None
+    default = default_choice(op, m, n, k)
     inherited[key] = default
     _VALIDATED[key] = [(0.0, default)]
     if m <= 4 or m > MAX_ROWS:
@@ -516,7 +559,7 @@ def _choice(op, x, weight, run, native, epilogue=_native.EPI_STORE, prologue=Fal
             register(key, m, traffic, options, lambda: _CHOICES[key],
                      lambda choice: _CHOICES.__setitem__(key, choice))
         else:
-            _CHOICES[key] = "native" if prefer_native(m) else None
+            _CHOICES[key] = default_choice(op, m, n, k)
     return _CHOICES[key]
 
 

@@ -47,7 +47,7 @@ def gate_up_swiglu(x, gate_up_weight, norm_weight=None, eps=1e-6, config=None, r
         raise ValueError("a residual needs the norm it feeds (norm_weight)")
     from torch.nn import functional as F
 
-    from kernels.linear import _as_config, _choice, _fusable, fused_project, linear, prefer_native
+    from kernels.linear import FLOW, _as_config, _choice, _fusable, fused_project, linear, norm_apart, prefer_native
     from kernels.rmsnorm import rms_norm
 
     shape = x.shape
@@ -56,18 +56,21 @@ def gate_up_swiglu(x, gate_up_weight, norm_weight=None, eps=1e-6, config=None, r
     n = gate_up_weight.shape[0]
     if n % 2:
         raise ValueError("gate_up_weight must stack gate and up rows: an even row count")
-    out = torch.empty((m, n // 2), device=x.device, dtype=torch.bfloat16)
     res = None if residual is None else residual.reshape(-1, shape[-1]).contiguous()
     summed = None if residual is None else torch.empty_like(res)
     if m == 0:
-        act = out.reshape(*shape[:-1], n // 2)
+        act = torch.empty((*shape[:-1], n // 2), device=x.device, dtype=torch.bfloat16)
         return act if residual is None else (act, summed.reshape(shape))
     if config is None and residual is None and _fusable(flat, gate_up_weight, norm_weight):
         # selected like a plain projection, under its own key (kernels/linear.py _choice)
         def run(choice, w, inp=flat):
             y = torch.empty((inp.shape[0], w.shape[0] // 2), device=inp.device, dtype=torch.bfloat16)
-            st = fused_project(inp, w, _native.EPI_SWIGLU, y, norm_weight, eps, config=_as_config(choice),
-                               sumsq=sumsq)
+            cfg, gain, sums = _as_config(choice), norm_weight, sumsq
+            if cfg is None and prefer_native(m) and k <= _native.FLOW_MAX_K:
+                cfg = FLOW  # the rows normalised apart unless they are short (norm_apart)
+                if gain is not None and norm_apart(m, k):
+                    inp, gain, sums = rms_norm(inp, gain, eps), None, None
+            st = fused_project(inp, w, _native.EPI_SWIGLU, y, gain, eps, config=cfg, sumsq=sums)
             return y if st == _native.FTK_OK else None
 
         def native(w, inp=flat):
@@ -77,9 +80,12 @@ def gate_up_swiglu(x, gate_up_weight, norm_weight=None, eps=1e-6, config=None, r
         if choice == "native":
             # the form selection timed: torch's GEMM itself, never a second selection by linear()
             return native(gate_up_weight).reshape(*shape[:-1], n // 2)
-        status = fused_project(flat, gate_up_weight, _native.EPI_SWIGLU, out, norm_weight, eps,
-                               config=_as_config(choice), sumsq=sumsq)
+        act = run(choice, gate_up_weight)
+        if act is not None:
+            return act.reshape(*shape[:-1], n // 2)
+        status = _native.FTK_ERR_UNSUPPORTED
     else:
+        out = torch.empty((m, n // 2), device=x.device, dtype=torch.bfloat16)
         status = _native.FTK_ERR_UNSUPPORTED if prefer_native(m, config) else \
             fused_project(flat, gate_up_weight, _native.EPI_SWIGLU, out, norm_weight, eps, residual=res,
                           summed=summed, config=config, sumsq=sumsq)

@@ -90,9 +90,11 @@ typedef enum ftk_kind {
                                weights loaded as 4 rows x 256 contiguous bytes per wave load */
   FTK_KIND_STAGE = 7,       /* M <= 16, K = 128 C KW: QUAD's weight loads staged through LDS into
                                16x16x32 MFMA tiles */
-  FTK_KIND_RING = 8         /* M = 1..16, K = 128 C KW: weight and x segments loaded straight into a
+  FTK_KIND_RING = 8,        /* M = 1..16, K = 128 C KW: weight and x segments loaded straight into a
                                per-wave LDS ring (global_load_lds_dwordx4), 16x16x32 MFMA tiles;
                                no residual-add prologue */
+  FTK_KIND_FLOW = 9         /* M = 1..32, any K % 8 == 0 up to 5120: RING's walk with the x rows in
+                               registers throughout; no residual add, in prologue or epilogue */
 } ftk_kind;
 
 /* Launch choice for one projection (the reference's per-shape config tuple,
@@ -104,19 +106,23 @@ typedef struct ftk_config {
                           MFMA: rows per workgroup (16, 32, 64); MFMA_STREAM, STAGE: rows per tile
                           (16, 32); QUAD: weight rows per row group per tile (4, 8, 16, 24; SwiGLU
                           8, 16, 24); RING: 16 (SwiGLU: 8 gate + 8 up rows), or for the
-                          STORE epilogue 12 (at K = 4096), or 24 (at up to 8 rows) */
+                          STORE epilogue 12 (at K = 4096), or 24 (at up to 8 rows);
+                          FLOW: 16, 8 (half of them gate rows for SwiGLU), or 12 (STORE) */
   int unroll;          /* GEMV: 16-byte chunks per lane per load batch (1, 2, 4);
-                          MFMA: K steps of loads in flight per wave (T = 1, 2: 4 or 8; T = 4: 2 or 4);
+                          MFMA: K steps of loads in flight per wave (T = 1, 2: 4 or 8; T = 4: 2 or 4), or
+                          1: the LDS-fed form (what a zero rows_per_wave, unroll and waves select):
+                          8, 12, 16, 20 or 24 rows with 8 waves, or 16, 24 or 32 with 4 (SwiGLU: 32);
                           STREAM, QUAD: unused (K fixes the chunks per lane);
                           MFMA_STREAM: K steps of weight loads in flight per wave (2, 4, 8);
                           STAGE: 128-wide K segments of weight loads in flight per wave (2..6);
-                          RING: units (K segments of a tile) in flight per wave (2; 3 at K = 12288) */
-  int groups_per_cu;   /* GEMV, STREAM, MFMA_STREAM, QUAD, STAGE, RING: grid cap = groups_per_cu * CUs (grid-stride
-                          beyond; the STREAM kinds raise the grid so no workgroup walks more tiles
+                          RING: units (K segments of a tile) in flight per wave (2; 3 at K = 12288);
+                          FLOW: unused */
+  int groups_per_cu;   /* GEMV, STREAM, MFMA_STREAM, QUAD, STAGE, RING, FLOW: grid cap =
+                          groups_per_cu * CUs (grid-stride beyond; the STREAM kinds raise the grid so no workgroup walks more tiles
                           than its LDS holds); MFMA: unused */
   int waves;           /* MFMA, MFMA_STREAM, STAGE, RING: waves per workgroup splitting K (4, 8, 16);
                           GEMV, STREAM: waves per row group splitting K (1, 2, 4, 8; a workgroup is
-                          4 waves, or 8 when 8 split K);
+                          4 waves, or 8 when 8 split K); FLOW: 8;
                           QUAD: waves per row group splitting K (4, 8, 16; the workgroup is
                           max(4, waves) waves) */
 } ftk_config;

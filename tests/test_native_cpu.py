@@ -530,3 +530,34 @@ def test_lm_head_plans_on_other_cu_counts(cus, m):
             assert p.workspace_bytes >= 128 + 4
         if m < 5:
             assert p.tiles >= 16 * cus
+
+
+@pytest.mark.parametrize("cus", [64, 256, 304])
+@pytest.mark.parametrize("m", [1, 4, 5, 16, 17, 32])
+def test_any_width_plans_write_every_output_once(m, cus):
+    """K that the STREAM, QUAD, STAGE and RING builds do not divide: FLOW and the MFMA kind's LDS-fed
+    form write every output once, whatever the CU count, and fit their argmax keys."""
+    for n, k in ((1, 8), (100, 136), (1926, 1000), (2560, 1920), (5000, 5120), (7000, 9728), (6144, 8192)) + \
+            (((512, 70000),) if m > 4 else ()):  # (below 5 rows the norm's x rows do not fit the LDS there)
+        for epi in (_native.EPI_STORE, _native.EPI_SWIGLU, _native.EPI_ARGMAX):
+            if epi == _native.EPI_SWIGLU and n % 2:
+                continue
+            for flags in (0, _native.PLAN_PROLOGUE):
+                p = _native.Plan()
+                assert _native.lib().ftk_plan_project(m, n, k, epi | flags, cus, None, p) == _native.FTK_OK
+                counts, max_row = _coverage(p, n, epi)
+                assert np.all(counts == 1) and max_row == n - 1, (n, k, epi, flags, p.kind)
+                if epi == _native.EPI_ARGMAX:
+                    assert p.workspace_bytes >= 256 + 8 * m * p.grid
+
+
+def test_default_choice_from_seventeen_rows():
+    from kernels import linear as L
+    assert all(L.default_choice(op, 16, 64, 32) is None for op in ("linear", "norm", "swiglu", "argmax"))
+    for op in ("linear", "norm", "swiglu", "argmax"):
+        assert L.default_choice(op, 20, 1536, 1024) == "native"  # a small weight
+        assert L.default_choice(op, 40, 4096, 4096) == "native"  # past MAX_ROWS
+        assert L.default_choice(op, 20, 4096, 4095) == "native"  # no fused kernel
+        assert L.default_choice(op, 20, 4096, 4096) is None
+    assert L.default_choice("linear", 20, 4096, 12288) is None and L.default_choice("linear", 20, 8192, 4096) == "native"
+    assert L.default_choice("swiglu", 20, 8192, 6144) == "native" and L.default_choice("norm", 20, 7168, 5120) is None
