@@ -78,6 +78,17 @@ __device__ __forceinline__ u32x2_t out_add4(const ProjArgs& a, int m, int n0) {
   return v;
 }
 
+// One residual element loaded ahead of its use (add_bits): an unconditional load, from x where there
+// is no residual, since a branch around a load ends in a join that waits for it.
+__device__ __forceinline__ uint32_t out_add1(const ProjArgs& a, int m, int n) {
+  const uint16_t* r = a.out_add != nullptr ? a.out_add + (size_t)m * a.N + n : a.x;
+  return *r;
+}
+__device__ __forceinline__ uint32_t add_bits(const ProjArgs& a, float s, uint32_t add) {
+  const uint32_t b = f32_to_bf16(s);
+  return a.out_add == nullptr ? b : f32_to_bf16(bf16_to_f32(b) + bf16_to_f32(add));
+}
+
 // store_bits of four outputs whose residual elements were loaded by out_add4.
 __device__ __forceinline__ void store_bits4(const ProjArgs& a, const f32x4_t& s, u32x2_t add, uint32_t (&bits)[4]) {
 #pragma unroll

@@ -278,6 +278,17 @@ __global__ __launch_bounds__(64 * KW) void ring_kernel(ProjArgs a, int tiles) {
     }
   };
 
+  // The residual elements of this thread's outputs in the first epilogue, ahead of the units: loaded
+  // where they were added they took four dependent round trips at the end of the walk (three
+  // Qwen3-8B layers at M = 5, the add in O and down: 207.6 us then, 205.8 now).
+  constexpr bool kAdd = EPI == EPI_STORE && !PRO;
+  u32x2_t add0 = {0u, 0u};
+  if constexpr (kAdd) {
+    const int ln = tid & 63, sub = (tid >> 6) % SUB, i = tid / (64 * SUB);
+    const int t = i < my_tiles ? tile_at(i) : 0;
+    add0 = out_add4(a, min(ln & 15, M - 1), t * RT + 16 * sub + 4 * (ln >> 4));
+  }
+
   // ---- RMSNorm prologue, part 1: the gain and the x rows (row-contiguous), issued
   // before the first units so that they return first (loads complete in order) --
   constexpr int GPT = PRO ? (GCH + 64 * KW - 1) / (64 * KW) : 1;
@@ -395,10 +406,10 @@ __global__ __launch_bounds__(64 * KW) void ring_kernel(ProjArgs a, int tiles) {
           u += part[i][w][0][(2 + h) * 16 + ll];
         }
         const int c0 = tl * 8 + 4 * h;
-        uint16_t* yr = a.y + (size_t)ll * outputs;
+        uint32_t bits[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (c0 + r < outputs) yr[c0 + r] = (uint16_t)swiglu_bf16(s[r], u[r]);
+        for (int r = 0; r < 4; ++r) bits[r] = swiglu_bf16(s[r], u[r]);
+        store_row4(a.y + (size_t)ll * outputs, c0, outputs, bits);
       }
     } else {
       // Subtile sub holds unit rows 16 sub + 4 gg + r; with 24-row tiles the second
@@ -409,30 +420,22 @@ __global__ __launch_bounds__(64 * KW) void ring_kernel(ProjArgs a, int tiles) {
         const int ll = ln & 15, gg = ln >> 4;
         if (ll >= M || 16 * sub + 4 * gg >= RT) continue;
         const int tl = flush_tile(done + i);
+        const int n0 = tl * RT + 16 * sub + 4 * gg;
+        u32x2_t add = add0;
+        if constexpr (kAdd) {
+          if (done != 0 || e >= 64 * KW) add = out_add4(a, ll, n0);
+        }
         f32x4_t s = part[i][0][sub][ln];
 #pragma unroll
         for (int w = 1; w < KW; ++w) s += part[i][w][sub][ln];
-        const int n0 = tl * RT + 16 * sub + 4 * gg;
         uint32_t bits[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          if constexpr (EPI == EPI_STORE)
-            bits[r] = n0 + r < a.N ? store_bits(a, s[r], ll, n0 + r) : 0u;
-          else
-            bits[r] = f32_to_bf16(s[r]);
-        }
-        if (a.y != nullptr) {
-          uint16_t* yr = a.y + (size_t)ll * a.N;
-          if (n0 + 3 < a.N && (a.N & 3) == 0 && (reinterpret_cast<uintptr_t>(a.y) & 7) == 0) {
-            *reinterpret_cast<u32x2_t*>(yr + n0) = u32x2_t{bits[0] | (bits[1] << 16), bits[2] | (bits[3] << 16)};
-          } else {
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-              if (n0 + r < a.N) yr[n0 + r] = (uint16_t)bits[r];
-          }
-        }
+        store_bits4(a, s, add, bits);
+        if (a.y != nullptr) store_row4(a.y + (size_t)ll * a.N, n0, a.N, bits);
         if constexpr (EPI == EPI_STORE && RT == 16) {
           if (a.sumsq_out != nullptr) {  // the entry's sum of squares waits in the slot it came from
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              if (n0 + r >= a.N) bits[r] = 0u;
             const float v0 = bf16_to_f32(bits[0]), v1 = bf16_to_f32(bits[1]);
             const float v2 = bf16_to_f32(bits[2]), v3 = bf16_to_f32(bits[3]);
             part[i][0][0][ln][0] = (v0 * v0 + v1 * v1) + (v2 * v2 + v3 * v3);
