@@ -1,209 +1,25 @@
 // Split-KV GQA decode attention on gfx950: engine/kernels/decode_attention.py:31-149
 // (_decode_partials, _decode_merge, _attend) and :229-258 (decode_attention).
 //
-// One workgroup per (row, KV head, split). The G query heads of a KV head
-// share every cache row the workgroup reads. A wave load covers 64 / (D / 8)
-// whole cache rows (4 rows x 256 bytes at D = 128): lane (r, c) holds the
-// 16-byte chunk c of row r, for K and for V. Per lane:
-//   - the G query slices of chunk c stay in registers;
-//   - each row's G scores are v_dot2 partial dots summed over the row's lanes
-//     by a DPP butterfly, so every lane of the row holds the same bits;
-//   - an online softmax runs over the rows the lane sees (max, denominator,
-//     and the numerator's 8 dimensions of chunk c per query head), with
-//     p rounded to BF16 before it multiplies V, as the reference's
-//     tl.dot(p.to(bf16), v) does; the denominator sums the FP32 p.
-// The rows of a wave, then the waves (through LDS), merge their softmax
-// states. One split writes the output; several write FP32 partials and
-// (max, denominator) pairs for the merge kernel. Slots at or past
-// min(position + 1, capacity) are never used: their scores are -inf and
-// their values are replaced by zero before any arithmetic (they may hold NaN).
+// One workgroup per (row, KV head, split), its interval an equal share of the
+// slots the row can see (min(position + 1, capacity)), so rows that stand at
+// different places of their caches keep all their workgroups busy. The G query
+// heads of a KV head share every cache row the workgroup reads. An online
+// softmax runs over the slots (max, denominator, numerator); p is rounded to
+// BF16 before it multiplies V, as the reference's tl.dot(p.to(bf16), v) does
+// (the tile kernel keeps the remainder too); the denominator sums the FP32 p. The waves (through LDS) merge their softmax
+// states; one split writes the output, several write FP32 partials and (max,
+// denominator) pairs for the merge kernel. Slots a row can't see are never
+// used: their scores are -inf and their values are replaced by zero before any
+// arithmetic (they may hold NaN).
+//
+// Two kernels: the tile kernel (ftk_attn_tile.hip, any shape) and QUAD below
+// (D = 128, up to 4 heads per KV head, short intervals); launch_attention holds the rule.
 #include "../../include/ftk.h"
+#include "ftk_attn.h"
 #include "ftk_internal.h"
 
 namespace ftk {
-
-// Sum over aligned groups of CH lanes (CH = 8 or 16). Every step adds a lane
-// pair in both orders, so all lanes of a group end with the same bits.
-template <int CH>
-__device__ __forceinline__ float group_sum(float v) {
-  v += dpp<0xB1, 0xF>(v);   // quad_perm [1,0,3,2]: lane ^ 1
-  v += dpp<0x4E, 0xF>(v);   // quad_perm [2,3,0,1]: lane ^ 2
-  v += dpp<0x141, 0xF>(v);  // row_half_mirror: lane ^ 7 within 8
-  if constexpr (CH == 16) v += dpp<0x140, 0xF>(v);  // row_mirror: lane ^ 15 within 16
-  return v;
-}
-
-__device__ __forceinline__ float exp2_f32(float x) { return __builtin_amdgcn_exp2f(x); }
-
-// Softmax state (max m, denominator l, numerator a) of one query head over 8 dimensions.
-template <int E>
-__device__ __forceinline__ void merge_state(float& m, float& l, float (&a)[E], float m2, float l2,
-                                            const float (&a2)[E]) {
-  const float top = fmaxf(m, m2);
-  const float pivot = top == -INFINITY ? 0.f : top;  // nothing seen on either side: keep zeros
-  const float c1 = exp2_f32(m - pivot), c2 = exp2_f32(m2 - pivot);
-  l = l * c1 + l2 * c2;
-#pragma unroll
-  for (int e = 0; e < E; ++e) a[e] = a[e] * c1 + a2[e] * c2;
-  m = top;
-}
-
-// A workgroup's merged state of query head h, dimensions 8 cc .. 8 cc + 7: the
-// output itself (one interval) or the interval's FP32 partial and (max, denominator).
-__device__ __forceinline__ void store_state(const AttnArgs& a, int group, int split, int h, int cc, int G, int D,
-                                            float m, float l, const float (&acc)[8]) {
-  if (a.splits == 1) {
-    uint32_t o[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] = pack_bf16(acc[2 * i] / l, acc[2 * i + 1] / l);
-    store16(a.out + ((size_t)group * G + h) * D + cc * 8, u32x4_t{o[0], o[1], o[2], o[3]});
-  } else {
-    const size_t slot = ((size_t)group * a.splits + split) * G + h;
-    float* dst = a.partial + slot * D + cc * 8;
-    *reinterpret_cast<f32x4_t*>(dst) = f32x4_t{acc[0], acc[1], acc[2], acc[3]};
-    *reinterpret_cast<f32x4_t*>(dst + 4) = f32x4_t{acc[4], acc[5], acc[6], acc[7]};
-    if (cc == 0) *reinterpret_cast<f32x2_t*>(a.stats + slot * 2) = f32x2_t{m, l};
-  }
-}
-
-template <int D, int G, int W, int U>
-__global__ __launch_bounds__(64 * W) void attn_partials_kernel(AttnArgs a) {
-  constexpr int CH = D / 8;     // 16-byte chunks per cache row
-  constexpr int RPL = 64 / CH;  // cache rows per wave load
-  constexpr int SLOTS = RPL * U;
-  __shared__ float acc_lds[W][G][D];
-  __shared__ float m_lds[W][G], l_lds[W][G];
-
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int r = lane / CH, c = lane - (lane / CH) * CH;
-  const int group = blockIdx.x / a.splits, split = blockIdx.x - group * a.splits;
-  const int row = group / a.kv_heads;
-  const int64_t newest = a.position[a.pos_stride * row];
-  const int64_t visible = newest + 1 < (int64_t)a.capacity ? newest + 1 : (int64_t)a.capacity;
-  const int begin = split * a.chunk;
-  const int end = (int)(begin + a.chunk < visible ? begin + a.chunk : visible);
-  const int units = end > begin ? (end - begin + SLOTS - 1) / SLOTS : 0;
-
-  const size_t cache = (size_t)group * a.capacity * D + c * 8;
-  const uint16_t* kb = a.k + cache;
-  const uint16_t* vb = a.v + cache;
-  u32x4_t qv[G];
-#pragma unroll
-  for (int h = 0; h < G; ++h) qv[h] = load16(a.q + ((size_t)group * G + h) * D + c * 8);
-
-  float m[G], l[G], acc[G][8];
-#pragma unroll
-  for (int h = 0; h < G; ++h) {
-    m[h] = -INFINITY;
-    l[h] = 0.f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) acc[h][e] = 0.f;
-  }
-
-  // Unit i covers slots begin + i SLOTS + [0, SLOTS); wave w takes units w, w + W, ...
-  // Rows past `end` load row end - 1 (inside the cache) and are masked below.
-  auto load_unit = [&](int unit, u32x4_t (&kr)[U], u32x4_t (&vr)[U]) {
-    const int first = begin + unit * SLOTS + r;
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int t = first + u * RPL < end ? first + u * RPL : end - 1;
-      kr[u] = load_stream16(kb + (size_t)t * D);
-      vr[u] = load_stream16(vb + (size_t)t * D);
-    }
-  };
-
-  u32x4_t kr[U], vr[U];
-  int unit = wave;
-  if (unit < units) load_unit(unit, kr, vr);
-  for (; unit < units; unit += W) {
-    u32x4_t kn[U], vn[U];
-    if (unit + W < units) load_unit(unit + W, kn, vn);
-
-    const int first = begin + unit * SLOTS + r;
-    float s[G][U];
-    float vf[U][8];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const bool live = first + u * RPL < end;
-#pragma unroll
-      for (int h = 0; h < G; ++h) {
-        const float dot = group_sum<CH>(dot8(kr[u], qv[h], 0.f));
-        s[h][u] = live ? dot * a.scale_log2 : -INFINITY;
-      }
-      const u32x4_t zero = {0u, 0u, 0u, 0u};
-      widen8(live ? vr[u] : zero, vf[u]);
-    }
-#pragma unroll
-    for (int h = 0; h < G; ++h) {
-      float top = m[h];
-#pragma unroll
-      for (int u = 0; u < U; ++u) top = fmaxf(top, s[h][u]);
-      const float pivot = top == -INFINITY ? 0.f : top;
-      const float corr = exp2_f32(m[h] - pivot);
-      float psum = 0.f;
-      float pb[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const float p = exp2_f32(s[h][u] - pivot);
-        psum += p;
-        pb[u] = round_bf16(p);
-      }
-      l[h] = l[h] * corr + psum;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        float v = acc[h][e] * corr;
-#pragma unroll
-        for (int u = 0; u < U; ++u) v += pb[u] * vf[u][e];
-        acc[h][e] = v;
-      }
-      m[h] = top;
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      kr[u] = kn[u];
-      vr[u] = vn[u];
-    }
-  }
-
-  // The RPL rows of the wave (lanes c, c + CH, ...), then the waves in order.
-#pragma unroll
-  for (int off = CH; off < 64; off <<= 1) {
-#pragma unroll
-    for (int h = 0; h < G; ++h) {
-      float a2[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) a2[e] = __shfl_xor(acc[h][e], off);
-      merge_state(m[h], l[h], acc[h], __shfl_xor(m[h], off), __shfl_xor(l[h], off), a2);
-    }
-  }
-  if (r == 0) {
-#pragma unroll
-    for (int h = 0; h < G; ++h) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) acc_lds[wave][h][c * 8 + e] = acc[h][e];
-      if (c == 0) {
-        m_lds[wave][h] = m[h];
-        l_lds[wave][h] = l[h];
-      }
-    }
-  }
-  __syncthreads();
-  const int t = threadIdx.x;
-  if (t < G * CH) {
-    const int h = t / CH, cc = t - (t / CH) * CH;
-    float mm = m_lds[0][h], ll = l_lds[0][h], aa[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) aa[e] = acc_lds[0][h][cc * 8 + e];
-#pragma unroll
-    for (int w = 1; w < W; ++w) {
-      float a2[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) a2[e] = acc_lds[w][h][cc * 8 + e];
-      merge_state(mm, ll, aa, m_lds[w][h], l_lds[w][h], a2);
-    }
-    store_state(a, group, split, h, cc, G, D, mm, ll, aa);
-  }
-}
 
 // ---- QUAD kind: D = 128, up to 4 query heads per KV head --------------------
 //
@@ -246,81 +62,13 @@ __device__ __forceinline__ float head_max(float v) {
   return fmaxf(v, __shfl_xor(v, 32));
 }
 
-// Lane l ^ 32's value: v_permlane32_swap trades lanes 32..63 of its first
-// operand with lanes 0..31 of its second; with both = v, the second comes
-// back holding v[l + 32] in lanes 0..31 and the first v[l - 32] in lanes 32..63.
-__device__ __forceinline__ float lane_xor32(float v, int lane) {
-  const unsigned u = __builtin_bit_cast(unsigned, v);
-  const auto p = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  return __builtin_bit_cast(float, lane < 32 ? p[1] : p[0]);
-}
-
-// Lane l ^ 16's value: v_permlane16_swap trades the odd 16-lane rows of its
-// first operand with the even rows of its second.
-__device__ __forceinline__ float lane_xor16(float v, int lane) {
-  const unsigned u = __builtin_bit_cast(unsigned, v);
-  const auto p = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  return __builtin_bit_cast(float, (lane & 16) ? p[0] : p[1]);
-}
-
-// Sum over the 16 lanes that share lane bits 0..1, the same bits in all of
-// them, on the VALU. row_ror:8 is lane ^ 8 inside a row of 16; its sum is the
-// same under ^ 8, so row_ror:4 (which reaches l ^ 4 or l ^ 12) adds lane ^ 4's
-// value. Every step adds a lane pair in both orders.
-__device__ __forceinline__ float quad_group_sum(float v, int lane) {
-  v += dpp<0x128, 0xF>(v);  // row_ror:8
-  v += dpp<0x124, 0xF>(v);  // row_ror:4
-  v += lane_xor16(v, lane);
-  return v + lane_xor32(v, lane);
-}
-
-// Head RMSNorm, gain and RoPE of one D = 128 head in the QUAD layout: lane
-// 4 c + i holds elements 8 c .. 8 c + 7 (c = 0..15), the 16 lanes of one i the
-// whole head; element j + 64 of element j's rotation is in chunk c ^ 8, lane ^ 32.
-// n = bf16(x / sqrt(mean(x^2) + eps)), w = bf16(n g),
-// out = bf16(bf16(w cos) + bf16(rotate_half(w) sin)) (engine/kernels/qk_rope.py:48-76).
-__device__ __forceinline__ u32x4_t quad_head_rope(u32x4_t x, u32x4_t g, u32x4_t c, u32x4_t s, float eps,
-                                                  int lane) {
-  float xf[8], gf[8], cf[8], sf[8];
-  widen8(x, xf);
-  widen8(g, gf);
-  widen8(c, cf);
-  widen8(s, sf);
-  float ss = 0.f;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) ss += xf[e] * xf[e];
-  ss = quad_group_sum(ss, lane);
-  const float inv_std = 1.0f / sqrtf(ss / 128.f + eps);
-  float w[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) w[e] = round_bf16(round_bf16(xf[e] * inv_std) * gf[e]);
-  uint32_t o[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    float r[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int e = 2 * i + j;
-      const float partner = lane_xor32(w[e], lane);
-      const float rot = lane < 32 ? -partner : partner;  // chunk < 8: the first half of the head
-      r[j] = round_bf16(w[e] * cf[e]) + round_bf16(rot * sf[e]);
-    }
-    o[i] = pack_bf16(r[0], r[1]);
-  }
-  return u32x4_t{o[0], o[1], o[2], o[3]};
-}
-
 // ROPE: the query heads are normalised and rotated here from the packed QKV
 // row, and the split whose interval holds the row's own slot (the position,
 // when it lies inside the cache) takes that slot's key and value from the
 // packed row too: it writes them to the cache, reads only the slots before
 // it from memory, and starts wave 0's softmax state with the new slot
 // (score s, p = 1). No other workgroup of the launch reads that slot.
-// FENCE (with ROPE): the head arithmetic is kept behind the first cache loads,
-// so it waits for the head loads only. That shortens a short split (the prologue
-// is most of it); in a long one the new slot's stores, then in flight ahead of
-// the loop, make the loop's waits drain more, so long splits go without.
-template <int G, int W, int NG, bool ROPE, bool FENCE = false>
+template <int G, int W, int NG, bool ROPE>
 __global__ __launch_bounds__(64 * W) void attn_quad_kernel(AttnArgs a) {
   constexpr int D = 128, SLOTS = 16 * NG;  // a unit: NG groups of 16 cache rows
   __shared__ float p_lds[W][64];
@@ -339,10 +87,13 @@ __global__ __launch_bounds__(64 * W) void attn_quad_kernel(AttnArgs a) {
     const int64_t loaded = *(a.phases != nullptr ? a.phases + row : a.position + a.pos_stride * row);
     shift = a.phases != nullptr ? loaded : 0;
   }
-  const int64_t visible = newest + 1 < (int64_t)a.capacity ? newest + 1 : (int64_t)a.capacity;
-  const int begin = split * a.chunk;
-  int end = (int)(begin + a.chunk < visible ? begin + a.chunk : visible);
-  bool own = ROPE && newest >= begin && newest < (int64_t)begin + a.chunk && newest < (int64_t)a.capacity;
+  const int64_t seen = newest + 1 < (int64_t)a.capacity ? newest + 1 : (int64_t)a.capacity;
+  const int64_t visible = seen > 0 ? seen : 0;
+  const int64_t slots = interval_slots(a, visible, SLOTS);
+  const int64_t begin64 = split * slots;
+  const int begin = (int)(begin64 < visible ? begin64 : visible);  // an interval past the row is empty
+  int end = (int)(begin64 + slots < visible ? begin64 + slots : visible);
+  bool own = ROPE && newest >= begin64 && newest < begin64 + slots && newest < (int64_t)a.capacity;
   if (own) end = (int)newest;
   const int units = end > begin ? (end - begin + SLOTS - 1) / SLOTS : 0;
   const u32x4_t zero = {0u, 0u, 0u, 0u};
@@ -401,7 +152,7 @@ __global__ __launch_bounds__(64 * W) void attn_quad_kernel(AttnArgs a) {
       vr[g][u] = buffer_load16(vrs, at(wave, g, u));
     }
   if constexpr (ROPE) {
-    if constexpr (FENCE) __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_sched_barrier(0);  // behind the cache loads: the prologue waits for the head loads only
     qv = quad_head_rope(xq, gq, cs, sn, a.q_eps, lane);
     if (i4 >= G) qv = zero;
     if (own) {
@@ -617,79 +368,35 @@ __global__ __launch_bounds__(64 * kMergeWaves) void attn_merge_kernel(const floa
   }
 }
 
-// Registers of one lane, estimated from the compiler's counts (gfx950): two unit
-// buffers of K and V plus the widened V rows (~18 per unit), query slice and
-// softmax state (~17 per head), scores (one per head and unit), addressing.
-constexpr bool attn_fits(int g, int u) { return 24 + 18 * u + 17 * g + g * u <= 230; }
-
-template <int D, int G, int W, int U>
-static hipError_t launch_partials(const AttnArgs& a, int grid, hipStream_t stream) {
-  if constexpr (attn_fits(G, U)) {
-    hipLaunchKernelGGL((attn_partials_kernel<D, G, W, U>), dim3((unsigned)grid), dim3(64 * W), 0, stream, a);
-    return hipGetLastError();
-  } else {
-    return hipErrorInvalidValue;
-  }
-}
-
-template <int D, int G>
-static hipError_t launch_for_group(const AttnArgs& a, const AttnShape& s, hipStream_t stream) {
-  const int grid = s.groups * s.splits;
-  if (s.waves == 4 && s.unroll == 2) return launch_partials<D, G, 4, 2>(a, grid, stream);
-  if (s.waves == 4 && s.unroll == 4) return launch_partials<D, G, 4, 4>(a, grid, stream);
-  if (s.waves == 4 && s.unroll == 8) return launch_partials<D, G, 4, 8>(a, grid, stream);
-  if (s.waves == 8 && s.unroll == 2) return launch_partials<D, G, 8, 2>(a, grid, stream);
-  if (s.waves == 8 && s.unroll == 4) return launch_partials<D, G, 8, 4>(a, grid, stream);
-  if (s.waves == 8 && s.unroll == 8) return launch_partials<D, G, 8, 8>(a, grid, stream);
-  return hipErrorInvalidValue;
-}
-
-template <int D>
-static hipError_t launch_for_dim(const AttnArgs& a, const AttnShape& s, hipStream_t stream) {
-  switch (s.group_size) {
-    case 1: return launch_for_group<D, 1>(a, s, stream);
-    case 2: return launch_for_group<D, 2>(a, s, stream);
-    case 3: return launch_for_group<D, 3>(a, s, stream);
-    case 4: return launch_for_group<D, 4>(a, s, stream);
-    case 5: return launch_for_group<D, 5>(a, s, stream);
-    case 6: return launch_for_group<D, 6>(a, s, stream);
-    case 7: return launch_for_group<D, 7>(a, s, stream);
-    case 8: return launch_for_group<D, 8>(a, s, stream);
-    default: return hipErrorInvalidValue;
-  }
-}
-
-template <int G, bool ROPE, bool FENCE>
+template <int G, bool ROPE>
 static hipError_t launch_quad_for_group(const AttnArgs& a, const AttnShape& s, hipStream_t stream) {
   const dim3 grid((unsigned)(s.groups * s.splits));
   if (s.waves == 4 && s.unroll == 1)
-    hipLaunchKernelGGL((attn_quad_kernel<G, 4, 1, ROPE, FENCE>), grid, dim3(256), 0, stream, a);
+    hipLaunchKernelGGL((attn_quad_kernel<G, 4, 1, ROPE>), grid, dim3(256), 0, stream, a);
   else if (s.waves == 4 && s.unroll == 2)
-    hipLaunchKernelGGL((attn_quad_kernel<G, 4, 2, ROPE, FENCE>), grid, dim3(256), 0, stream, a);
+    hipLaunchKernelGGL((attn_quad_kernel<G, 4, 2, ROPE>), grid, dim3(256), 0, stream, a);
   else if (s.waves == 8 && s.unroll == 1)
-    hipLaunchKernelGGL((attn_quad_kernel<G, 8, 1, ROPE, FENCE>), grid, dim3(512), 0, stream, a);
+    hipLaunchKernelGGL((attn_quad_kernel<G, 8, 1, ROPE>), grid, dim3(512), 0, stream, a);
   else if (s.waves == 8 && s.unroll == 2)
-    hipLaunchKernelGGL((attn_quad_kernel<G, 8, 2, ROPE, FENCE>), grid, dim3(512), 0, stream, a);
+    hipLaunchKernelGGL((attn_quad_kernel<G, 8, 2, ROPE>), grid, dim3(512), 0, stream, a);
   else
     return hipErrorInvalidValue;
   return hipGetLastError();
 }
 
-template <bool ROPE, bool FENCE>
+template <bool ROPE>
 static hipError_t launch_quad(const AttnArgs& a, const AttnShape& s, hipStream_t stream) {
   switch (s.group_size) {
-    case 1: return launch_quad_for_group<1, ROPE, FENCE>(a, s, stream);
-    case 2: return launch_quad_for_group<2, ROPE, FENCE>(a, s, stream);
-    case 3: return launch_quad_for_group<3, ROPE, FENCE>(a, s, stream);
-    case 4: return launch_quad_for_group<4, ROPE, FENCE>(a, s, stream);
+    case 1: return launch_quad_for_group<1, ROPE>(a, s, stream);
+    case 2: return launch_quad_for_group<2, ROPE>(a, s, stream);
+    case 3: return launch_quad_for_group<3, ROPE>(a, s, stream);
+    case 4: return launch_quad_for_group<4, ROPE>(a, s, stream);
     default: return hipErrorInvalidValue;
   }
 }
 
-// Splits of up to this many slots take the RoPE prologue with the scheduling fence
-// (measured on MI355X: B = 1 x 4K slots in 128-slot splits gains ~1 us with it;
-// 1024- and 2048-slot splits lose 1-3.5 us).
-constexpr int kAttnFenceMaxChunk = 256;
+// Which configurations of the ROWS kind a caller may name (heads per group and cache rows in flight).
+constexpr bool attn_fits(int g, int u) { return 24 + 18 * u + 17 * g + g * u <= 230; }
 
 bool attn_supported(int kind, int dim, int group_size, int waves, int unroll) {
   if (waves != 4 && waves != 8) return false;
@@ -704,12 +411,20 @@ bool attn_supported(int kind, int dim, int group_size, int waves, int unroll) {
 hipError_t launch_attention(const AttnArgs& a, const AttnShape& s, hipStream_t stream) {
   // The head norm + RoPE prologue exists for the QUAD kind only (the caller checks).
   if (a.packed != nullptr && s.kind != FTK_ATTN_QUAD) return hipErrorInvalidValue;
-  const bool rope = a.packed != nullptr, fence = s.chunk <= kAttnFenceMaxChunk;
-  hipError_t e = s.kind == FTK_ATTN_QUAD ? (!rope   ? launch_quad<false, false>(a, s, stream)
-                                            : fence ? launch_quad<true, true>(a, s, stream)
-                                                    : launch_quad<true, false>(a, s, stream))
-                 : s.dim == 128          ? launch_for_dim<128>(a, s, stream)
-                                         : launch_for_dim<64>(a, s, stream);
+  AttnArgs args = a;
+  args.group_size = s.group_size;
+  int log = 0;  // ceil(log2 splits)
+  while ((1 << log) < s.splits) ++log;
+  args.split_magic = (uint32_t)(((uint64_t)1 << (31 + log)) / s.splits + 1);
+  args.split_shift = 31 + log;
+  // A wave with at most one 32-slot unit even at a full cache has nothing to pipeline, and the way through
+  // LDS is then pure latency: QUAD keeps those (QKV rows, 8 KV heads x 4: B = 1 x 4K slots in 128-slot
+  // intervals 10.9 us against 11.7, 1K in 64-slot intervals 9.1 against 9.6). From two units on the tile
+  // kernel leads (256-slot intervals 12.0 against 12.9, 512-slot ones 14.0 against 16.5).
+  const bool quad = s.kind == FTK_ATTN_QUAD && s.chunk <= kTileSlots * s.waves;
+  hipError_t e = !quad                 ? launch_attn_tile(args, s, stream)
+                 : a.packed != nullptr ? launch_quad<true>(args, s, stream)
+                                       : launch_quad<false>(args, s, stream);
   if (e != hipSuccess || s.splits == 1) return e;
   const unsigned heads = (unsigned)(s.groups * s.group_size);
   if (s.dim == 128)

@@ -604,6 +604,13 @@ static int64_t call_workspace(const ftk_plan& p, int epi, bool pro) {
 // Workgroups the default split count aims at: one per CU (measured on MI355X:
 // 32 intervals per KV head beat 64 at B = 1 from 1K to 32K slots).
 constexpr int kAttnGroupsPerCu = 1;
+// Several rows over caches of more than 4K slots: intervals of 1K slots, up to four workgroups per CU, so
+// that rows standing at different places of their caches even out (8 KV heads x 4, positions spread over
+// 10%..100% of the cache: 16 x 8K 73.5 -> 57.4 us with 8 intervals instead of 2, 64.8 with 2; 32 x 8K 133 ->
+// 105; 4 x 16K 42 -> 34; 512-slot intervals and shorter lose again, 4 x 16K 35). At 4K slots the extra
+// intervals gain under 1% (16 rows: 51.4 -> 51.0 us).
+constexpr int kAttnGroupsPerCuLong = 4;
+constexpr int64_t kAttnLongSlots = 4096, kAttnLongChunk = 1024;
 
 static int attn_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t C, int64_t D, int cus, const ftk_attn_config* cfg,
                      ftk_attn_plan* p, AttnShape* shape) {
@@ -629,7 +636,13 @@ static int attn_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t C, int64_t D, i
     splits = cfg->splits < C ? cfg->splits : C;
     if (splits > kAttnMaxSplits) return FTK_ERR_INVALID;
   } else {
-    const int64_t want = ((int64_t)kAttnGroupsPerCu * cus + groups - 1) / groups;
+    auto share = [&](int per_cu) { return ((int64_t)per_cu * cus + groups - 1) / groups; };
+    int64_t want = share(kAttnGroupsPerCu);
+    if (B > 1 && C > kAttnLongSlots) {
+      const int64_t many = share(kAttnGroupsPerCuLong), whole = C / kAttnLongChunk;
+      const int64_t longer = many < whole ? many : whole;
+      if (longer > want) want = longer;
+    }
     const int64_t most = (C + waves * unit - 1) / (waves * unit);  // at least one step per wave
     splits = want < most ? want : most;
     if (splits > kAttnMaxSplits) splits = kAttnMaxSplits;
@@ -1208,7 +1221,6 @@ static int run_attention(AttnArgs& a, const void* k, const void* v, const int64_
   a.q_heads = (int)q_heads;
   a.capacity = (int)capacity;
   a.splits = p.splits;
-  a.chunk = p.chunk;
   a.scale_log2 = (float)(scale * 1.4426950408889634);
   return hip_status(launch_attention(a, shape, reinterpret_cast<hipStream_t>(stream)));
 }

@@ -376,8 +376,11 @@ struct AttnArgs {
   float* partial;           // [groups, splits, G, D] FP32 numerators (splits > 1 only)
   float* stats;             // [groups, splits, G, 2] FP32 (max, denominator) (splits > 1 only)
   int kv_heads;
+  int group_size;           // G: query heads per KV head
   int capacity;             // cache slots per group
-  int splits, chunk;        // slot intervals per group and slots per interval
+  int splits;               // slot intervals per group
+  uint32_t split_magic;     // n / splits = n split_magic >> split_shift (n < 2^31)
+  int split_shift;
   float scale_log2;         // scale * log2(e), formed in double
   // Q/K head norm + RoPE in the QUAD kind's prologue (rope_attention): q is
   // unused; query, key and value heads come from the packed QKV rows, and the
@@ -402,9 +405,9 @@ struct AttnShape {
   int group_size;  // G: query heads per KV head (1..kAttnMaxGroup)
   int groups;      // rows * KV heads
   int splits;      // slot intervals per group (1: the partials kernel writes the output)
-  int chunk;       // slots per interval
+  int chunk;       // slots per interval at a full cache
   int waves;       // W: waves per workgroup (4, 8)
-  int unroll;      // U: cache-row loads of K (and of V) in flight per lane (2, 4, 8)
+  int unroll;      // QUAD: groups of 16 cache rows per wave step (1, 2)
 };
 constexpr int kAttnMaxGroup = 8;
 constexpr int kAttnMaxSplits = 1024;  // slot intervals per group the merge kernel takes

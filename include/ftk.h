@@ -314,23 +314,23 @@ int64_t ftk_argmax_workspace_bytes(int64_t rows, int64_t vocab);
  * Zero fields mean "planner default". */
 typedef enum ftk_attn_kind {
   FTK_ATTN_AUTO = 0,
-  FTK_ATTN_ROWS = 1,  /* any D in {64, 128}, up to 8 query heads per KV head: v_dot2 scores summed
-                         over each cache row's lanes, an online softmax per lane, p V on the VALU */
+  FTK_ATTN_ROWS = 1,  /* any D in {64, 128}, up to 8 query heads per KV head: scores and p V on
+                         16x16x32 MFMAs, 32 slots of K and V per wave step through LDS */
   FTK_ATTN_QUAD = 2   /* D = 128, up to 4 query heads per KV head: scores on 16-block 4x4x4 MFMAs fed
                          by 4 cache rows x 256 bytes per wave load, one softmax step per (row, head),
-                         p V on the VALU */
+                         p V on the VALU; intervals of more than 32 slots per wave take ROWS' kernel */
 } ftk_attn_kind;
 typedef struct ftk_attn_config {
   int kind;    /* ftk_attn_kind */
   int splits;  /* slot intervals per (row, KV head), at most 1024; 1 = no merge launch */
   int waves;   /* waves per workgroup (4, 8) */
-  int unroll;  /* ROWS: cache rows of K (and of V) in flight per lane per step (2, 4, 8);
+  int unroll;  /* ROWS: 2, 4, 8 (8 with up to 2 heads), the same launch; sizes the default split count;
                   QUAD: groups of 16 cache rows per wave step, the loads of the next step in flight (1, 2) */
 } ftk_attn_config;
 typedef struct ftk_attn_plan {
   int kind;
   int splits;               /* slot intervals per (row, KV head) */
-  int chunk;                /* slots per interval */
+  int chunk;                /* slots per interval at a full cache; a row's intervals share its own slots */
   int waves;
   int unroll;
   int grid;                 /* partials workgroups: rows * KV heads * splits */

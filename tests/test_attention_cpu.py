@@ -154,3 +154,11 @@ def test_wrapper_keeps_the_reference_assertions():
         A.decode_attention(*_args(hq=18, hkv=2), 0.125)
     with pytest.raises(ValueError, match="GPU"):
         A.decode_attention(q, k, v, pos, 0.125)  # CPU tensors: no fallback
+
+
+@pytest.mark.parametrize("b,hkv,c,splits", [(16, 8, 4096, 2), (16, 8, 4097, 4), (16, 8, 8192, 8), (32, 8, 8192, 4),
+                                            (4, 8, 16384, 16), (8, 2, 8192, 16), (1, 8, 32768, 32), (300, 8, 8192, 1)])
+def test_several_rows_over_long_caches_take_intervals_of_1k_slots(b, hkv, c, splits):
+    """At most four workgroups per CU, and never fewer intervals than one workgroup per CU asks for."""
+    p = plan(b, 4 * hkv, hkv, c, 128)
+    assert p.splits == splits and p.chunk == -(-c // splits)
