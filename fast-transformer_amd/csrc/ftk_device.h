@@ -27,18 +27,11 @@ __device__ __forceinline__ float bf16_to_f32(uint32_t bits16) {
 __device__ __forceinline__ float lo_f32(uint32_t pair) { return __uint_as_float(pair << 16); }
 __device__ __forceinline__ float hi_f32(uint32_t pair) { return __uint_as_float(pair & 0xFFFF0000u); }
 
-__device__ __forceinline__ uint32_t f32_to_bf16(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7FFFFFFFu) > 0x7F800000u) return 0x7FC0u;
-  u += 0x7FFFu + ((u >> 16) & 1u);
-  return u >> 16;
-}
-
 // Two FP32 values rounded to nearest-even BF16, packed (lo in the low half),
 // by the compiler's float -> bfloat conversion (one v_cvt_pk_bf16_f32 on
 // gfx950). Finite values and infinities round exactly as f32_to_bf16; a NaN
 // stays a NaN with an unspecified payload, so this is only for values that
-// feed further arithmetic: stored results go through f32_to_bf16.
+// feed further arithmetic: stored results go through f32_to_bf16 or pack_bf16.
 __device__ __forceinline__ uint32_t rne_pair(float lo, float hi) {
   const f32x2_t v = {lo, hi};
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
@@ -47,10 +40,16 @@ __device__ __forceinline__ uint32_t rne_pair(float lo, float hi) {
 // FP32 -> nearest BF16 value, kept in FP32 (one rounding; an intermediate).
 __device__ __forceinline__ float round_bf16(float f) { return lo_f32(rne_pair(f, 0.f)); }
 
-// A stored BF16 pair: round-to-nearest-even, every NaN as 0x7FC0.
-__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
-  return f32_to_bf16(lo) | (f32_to_bf16(hi) << 16);
-}
+// The one NaN that is stored (0x7FC0 once rounded) in place of any other.
+__device__ __forceinline__ float stored_nan(float f) { return f != f ? __uint_as_float(0x7FC00000u) : f; }
+
+// A stored BF16 pair: round-to-nearest-even, every NaN as 0x7FC0. Through the conversion instruction a
+// pair takes 5 instructions; rounding by integer arithmetic took 11, and at a prompt's rows the row-wise
+// operators are bound by their instructions as much as by memory.
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) { return rne_pair(stored_nan(lo), stored_nan(hi)); }
+
+// One stored value, in the low half.
+__device__ __forceinline__ uint32_t f32_to_bf16(float f) { return pack_bf16(f, 0.f); }
 
 __device__ __forceinline__ bf16x2_t as_bf16x2(uint32_t v) { return __builtin_bit_cast(bf16x2_t, v); }
 
@@ -266,13 +265,16 @@ __device__ __forceinline__ float silu_f32(float g) {
   return g / (1.0f + expf(-g));
 }
 
-// SwiGLU on FP32 sums: gate and up are rounded to BF16 first, SiLU's output is
-// rounded to BF16, and the product is rounded once more (engine/kernels/swiglu.py:20-24).
+// SwiGLU of two outputs' gate and up values, BF16 already: SiLU's output is rounded to BF16 and the
+// products are rounded once more (engine/kernels/swiglu.py:20-24).
+__device__ __forceinline__ uint32_t swiglu_pair(float g0, float u0, float g1, float u1) {
+  const uint32_t a = rne_pair(silu_f32(g0), silu_f32(g1));
+  return pack_bf16(lo_f32(a) * u0, hi_f32(a) * u1);
+}
+
+// SwiGLU on one output's FP32 sums: gate and up are rounded to BF16 first.
 __device__ __forceinline__ uint32_t swiglu_bf16(float gate_sum, float up_sum) {
-  const float g = round_bf16(gate_sum);
-  const float u = round_bf16(up_sum);
-  const float a = round_bf16(silu_f32(g));
-  return f32_to_bf16(a * u);
+  return f32_to_bf16(round_bf16(silu_f32(round_bf16(gate_sum))) * round_bf16(up_sum));
 }
 
 }  // namespace ftk
