@@ -44,6 +44,7 @@ MAX_ROWS = _native.MAX_ROWS
 #: "native" = torch's GEMM (keep_native), or a launch tuple. _VALIDATED: the timed candidates.
 _CHOICES = {}
 _VALIDATED = {}
+_UNSELECTED = object()
 #: Time the candidate launch shapes of each shape at its first eager use, as linear.py:494-511
 #: always does. On by default; FTK_TUNE=0 (or ``TUNE = False``) keeps the planner's defaults, which
 #: come from the same kind of timing, done once on MI355X.
@@ -106,7 +107,7 @@ def _fusable(flat, weight, norm_weight=None):
 
 def _as_rows(x):
     rows = x.numel() // x.shape[-1]
-    return x.reshape(rows, x.shape[-1]).contiguous()
+    return x if x.dim() == 2 and x.is_contiguous() else x.reshape(rows, x.shape[-1]).contiguous()
 
 
 class SumSq:
@@ -655,15 +656,16 @@ def _linear(x, weight, sumsq):
     if rows == 0:
         return x.new_empty((*x.shape[:-1], weight.shape[0]))
     flat = _as_rows(x)
+    choice = _CHOICES.get(_key("linear", x.device, rows, weight.shape[0], x.shape[-1]), _UNSELECTED)
+    if choice is _UNSELECTED:
+        def run(choice, w, inp=flat):
+            return project(inp, w, _as_config(choice))
 
-    def run(choice, w, inp=flat):
-        return project(inp, w, _as_config(choice))
-
-    choice = _choice("linear", flat, weight, run, lambda w, inp=flat: F.linear(inp, w))
+        choice = _choice("linear", flat, weight, run, lambda w, inp=flat: F.linear(inp, w))
     if choice == "native":
         return F.linear(x, weight)
     out = project(flat, weight, _as_config(choice), sumsq=sumsq)
-    return out.reshape(*x.shape[:-1], weight.shape[0])
+    return out if x.dim() == 2 else out.reshape(*x.shape[:-1], weight.shape[0])
 
 
 def plan(m, n, k, epilogue=_native.EPI_STORE, compute_units=256, config=None, prologue=False, residual=False):
