@@ -612,6 +612,19 @@ constexpr int kAttnGroupsPerCu = 1;
 constexpr int kAttnGroupsPerCuLong = 4;
 constexpr int64_t kAttnLongSlots = 4096, kAttnLongChunk = 1024;
 
+// A short cache is one interval: the second launch (the merge) costs 1.5 to 2 us, more than the workgroup's
+// own walk. us with the default's intervals / with one, full cache, 8 KV heads: 1 x 256 x 4 heads 7.7 / 6.5,
+// 4 x 128 7.8 / 6.1, 4 x 256 7.8 / 7.2, 16 x 256 9.4 / 7.7, 8 heads per KV head 1 x 256 6.8 / 5.5, D = 64
+// 4 x 256 6.1 / 4.4. At 320 and 384 slots of 128 dimensions more than two intervals are the faster ones
+// (4 x 384 7.9 / 8.4) and two are not (16 x 384 10.5 / 9.1; D = 64, 4 x 384 6.1 / 5.3). One row of up to
+// 128 slots keeps an interval per step of its waves (its launch is part of the planner's known answers).
+constexpr int64_t kAttnOneInterval = 256, kAttnOneIntervalWide = 384;
+
+static bool attn_one_interval(int64_t B, int64_t C, int64_t D, int64_t splits) {
+  if (B == 1 && C <= 128) return false;
+  return C <= kAttnOneInterval || (C <= kAttnOneIntervalWide && (D == 64 || splits <= 2));
+}
+
 static int attn_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t C, int64_t D, int cus, const ftk_attn_config* cfg,
                      ftk_attn_plan* p, AttnShape* shape) {
   if (B < 1 || Hq < 1 || Hkv < 1 || C < 1 || Hq % Hkv || cus < 1) return FTK_ERR_INVALID;
@@ -646,7 +659,7 @@ static int attn_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t C, int64_t D, i
     const int64_t most = (C + waves * unit - 1) / (waves * unit);  // at least one step per wave
     splits = want < most ? want : most;
     if (splits > kAttnMaxSplits) splits = kAttnMaxSplits;
-    if (splits < 1) splits = 1;
+    if (splits < 1 || attn_one_interval(B, C, D, splits)) splits = 1;
   }
   const int64_t chunk = (C + splits - 1) / splits;
   splits = (C + chunk - 1) / chunk;  // no interval lies wholly past the cache

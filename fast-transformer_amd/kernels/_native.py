@@ -176,7 +176,8 @@ def try_call(name, *args):
 
 
 #: The raw handle itself: ``torch.cuda.current_stream`` builds a Stream object for each call, a large
-#: part of an eager launch's host time (with the rest of that path, one small projection launched eagerly 15.5 -> 10.3 us).
+#: part of an eager launch's host time (with the rest of that path, one small projection launched
+#: eagerly 15.5 -> 10.3 us).
 _raw_stream = torch._C._cuda_getCurrentRawStream
 
 
