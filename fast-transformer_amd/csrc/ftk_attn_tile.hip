@@ -10,10 +10,11 @@
 // columns (up to 8 of 16): a lane's four accumulators are one head's scores of
 // four slots, so the softmax needs two cross-lane steps per unit. p is already
 // in the B operand's layout of the second product, and ds_read_b64_tr_b16 gives
-// V's columns as its A operand; p goes in as two BF16 addends (16 bits of it,
-// where one rounding keeps 8), since the matrix cores are idle most of the time. The cost per unit does
-// not depend on the number of heads: with dot products and p V on the VALU it
-// grew with it and passed the loads' time from 5 heads per KV head on.
+// V's columns as its A operand; p goes in as two BF16 addends of one sign (16
+// bits of it, where one rounding keeps 8), since the matrix cores are idle most
+// of the time. The cost per unit does not depend on the number of heads: with
+// dot products and p V on the VALU it grew with it and passed the loads' time
+// from 5 heads per KV head on.
 // Measured (partials + merge): 1 x 32K slots, 8 KV heads x 8, 71.1 -> 29.2 us;
 // D = 64 x 4 heads 24.4 -> 16.7; 8 x 2K ragged, 8 heads, 39.4 -> 15.2; 16 x 8K
 // ragged, 4 heads, 72.9 -> 57.3 (8 intervals); 1 x 32K, 4 heads, 28.8 both.
@@ -88,6 +89,13 @@ __device__ __forceinline__ float quarter_max(float v) {
   const Pair r = row_pairs(v);
   const Pair h = halves(fmaxf(r.a, r.b));
   return fmaxf(h.a, h.b);
+}
+
+// What p's upper 16 bits leave of it, at least the smallest normal number where p is positive. That floor
+// adds 2^-126 to weights of up to 1; the largest finite value times it is 4.
+__device__ __forceinline__ float low_part(float p) {
+  const float rest = p - __uint_as_float(__float_as_uint(p) & 0xFFFF0000u);
+  return p > 0.f ? fmaxf(rest, 0x1p-126f) : 0.f;
 }
 
 }  // namespace
@@ -259,14 +267,15 @@ __global__ __launch_bounds__(64 * W) void attn_tile_kernel(AttnArgs a) {
     l = l * corr + sum;
     m = top;
     // p as two BF16 addends, the second product's operands: element e of quarter g is slot 4 g + e of tile 0,
-    // then of tile 1.
+    // then of tile 1. Neither is negative, and where p is not zero neither is zero (low_part): an infinite
+    // value then gives that infinity twice over, where 0 x inf or inf - inf would be no number. (Rounding
+    // p to nearest and adding what is left with its sign, without that property, takes as long.)
     u32x4_t ph, pl;
 #pragma unroll
     for (int h = 0; h < 4; ++h) {
       const float p0 = p[h >> 1][2 * (h & 1)], p1 = p[h >> 1][2 * (h & 1) + 1];
-      const uint32_t hi = rne_pair(p0, p1);
-      ph[h] = hi;
-      pl[h] = rne_pair(p0 - lo_f32(hi), p1 - hi_f32(hi));
+      ph[h] = __builtin_amdgcn_perm(__float_as_uint(p1), __float_as_uint(p0), 0x07060302u);
+      pl[h] = rne_pair(low_part(p0), low_part(p1));
     }
     if (__any(corr != 1.f)) {
 #pragma unroll
