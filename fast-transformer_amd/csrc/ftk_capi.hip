@@ -266,6 +266,9 @@ static bool flow_fits(int64_t M, int epi, bool pro, int64_t K) {
 // 6144 x 4096 (24 rows) 10.7 / 12.3 against 13.0 / 16.2. 24-row tiles of 25..32 x rows fit the LDS
 // with four waves only. Past 24 rows per CU two smaller workgroups share a CU: 16 rows
 // (8192 x 4096, M = 8: 14.3 against 16.5 with 32), 32 from 17 x rows (M = 32: 17.9 against 18.3).
+// Argmax from 17 x rows takes 32 too: half the key words, and the faster ones at most vocabularies
+// (24 rows, no norm: 151936 x 4096 253 against 311 with 16, 50257 x 6144 129 / 161, 32000 x 8192 114 /
+// 121, 8000 x 8192 36.0 / 35.1).
 struct MfmaLdsDefault {
   int rows, kw;
 };
@@ -279,9 +282,11 @@ static MfmaLdsDefault mfma_lds_default(int64_t M, int epi, bool pro, int64_t N, 
           if (fits(rows, kw)) return {rows, kw};
     if (M > 16 && fits(32, 4)) return {32, 4};
   }
-  if (epi == FTK_EPI_ARGMAX && fits(16, 8)) return {16, 8};
+  if (epi == FTK_EPI_ARGMAX && M > 16 && fits(32, 4)) return {32, 4};
+  if (epi == FTK_EPI_ARGMAX && M <= 16 && fits(16, 8)) return {16, 8};
   // (A norm's gain beside the rings: long rows leave room for the smaller workgroups only, or none.)
   const int rows = epi == FTK_EPI_SWIGLU ? 32 : 16;
+  if (epi == FTK_EPI_ARGMAX && M > 16) return {0, 0};  // the register-fed form's 32-row tiles
   return fits(rows, 4) ? MfmaLdsDefault{rows, 4} : MfmaLdsDefault{0, 0};
 }
 
@@ -1127,9 +1132,7 @@ int ftk_lm_head_argmax_static_bf16(const void* x, const void* gamma, float eps, 
   if (st != FTK_OK) return st;
   // Every key slot the finalize pass reads is written earlier in the same call,
   // so the array needs no clearing between calls.
-  // From 17 rows the bound is one key per row and 16-row tile, whatever the launch needs.
-  const int64_t keys = M > 16 ? argmax_keys_bytes((int)((V + 15) / 16), M) : call_workspace(p, FTK_EPI_ARGMAX, gamma != nullptr);
-  if (keys > FTK_STATIC_SCRATCH_BYTES) return FTK_ERR_TOO_LARGE;
+  if (call_workspace(p, FTK_EPI_ARGMAX, gamma != nullptr) > FTK_STATIC_SCRATCH_BYTES) return FTK_ERR_TOO_LARGE;
   void* ws = nullptr;
   const int got = static_scratch(&ws);
   if (got != FTK_OK) return got;

@@ -194,9 +194,10 @@ int ftk_lm_head_argmax_bf16(const void* x, const void* gamma, float eps, const v
  * the per-workgroup argmax keys live in a static device array of FTK_STATIC_SCRATCH_BYTES
  * (1 MiB) that every GPU the library runs on holds until the process ends. The array starts
  * zeroed and every call leaves its key words zero, as the workspace convention above asks.
- * Results are those of ftk_lm_head_argmax_bf16 bit for bit (same kernels). A call that needs
- * more keys than the array
- * holds (e.g. 32 rows of a 151936-entry vocabulary) returns FTK_ERR_TOO_LARGE and launches nothing.
+ * Results are those of ftk_lm_head_argmax_bf16 bit for bit (same kernels). A call whose launch
+ * needs more keys than the array holds (more than 27 rows of a 151936-entry vocabulary without
+ * gamma; with gamma and K up to 5120 the keys of 32 rows fit) returns FTK_ERR_TOO_LARGE and
+ * launches nothing.
  * Every call on one GPU shares that GPU's array: calls that overlap on one GPU (two streams, two
  * threads) race and give wrong ids; keep them in one stream. */
 int ftk_lm_head_argmax_static_bf16(const void* x, const void* gamma, float eps, const void* w, void* logits,
