@@ -56,7 +56,7 @@ def lm_head_argmax(x, weight, norm_weight=None, eps=1e-6, logits=True, top=None,
         raise ValueError("a residual needs the norm it feeds (norm_weight)")
     from torch.nn import functional as F
 
-    from kernels.linear import _as_config, _choice, _fusable, fused_project, linear, prefer_native
+    from kernels.linear import FLOW, _as_config, _choice, _fusable, fused_project, linear, prefer_native
     from kernels.rmsnorm import add_rms_norm, rms_norm
 
     shape = x.shape
@@ -73,12 +73,22 @@ def lm_head_argmax(x, weight, norm_weight=None, eps=1e-6, logits=True, top=None,
     if config is None and residual is None and _fusable(flat, weight, norm_weight):
         # selected like a plain projection, under its own key (kernels/linear.py _choice); the
         # agreement check compares the logits
+        def launch(choice, w, inp, lg, tok, top=None):
+            cfg, gain, sums = _as_config(choice), norm_weight, sumsq
+            if cfg is None and prefer_native(m) and k <= _native.FLOW_MAX_K:
+                # From 17 rows the walk, without a norm too (24 rows, us, against the tile form and the
+                # native GEMM + argmax: 151936 x 1024 57 / 75 / 78, 151936 x 4096 198 / 253 / 275, 32000 x
+                # 5120 57 / 63 / 65). Past K = 4096 its normalising builds spill registers, and the norm
+                # runs apart (32000 x 5120 60 against 73 fused, native 69; 75968 x 5120 133 / 155 / 178).
+                cfg = FLOW
+                if gain is not None and k > 4096:
+                    inp, gain, sums = rms_norm(inp, gain, eps), None, None
+            return fused_project(inp, w, _native.EPI_ARGMAX, lg, gain, eps, ids=tok, top=top, config=cfg, sumsq=sums)
+
         def run(choice, w, inp=flat):
             lg = torch.empty((inp.shape[0], w.shape[0]), device=inp.device, dtype=torch.bfloat16)
             tok = torch.empty((inp.shape[0],), device=inp.device, dtype=ids_dtype)
-            st = fused_project(inp, w, _native.EPI_ARGMAX, lg, norm_weight, eps, ids=tok, config=_as_config(choice),
-                               sumsq=sumsq)
-            return lg if st == _native.FTK_OK else None
+            return lg if launch(choice, w, inp, lg, tok) == _native.FTK_OK else None
 
         def native_logits(w, inp=flat):
             return F.linear(inp if norm_weight is None else rms_norm(inp, norm_weight, eps), w)
@@ -92,8 +102,7 @@ def lm_head_argmax(x, weight, norm_weight=None, eps=1e-6, logits=True, top=None,
             # the form selection timed: torch's GEMM itself, never a second selection by linear()
             full = native_logits(weight)
             return argmax(full, top=top).to(ids_dtype), (full.reshape(*shape[:-1], v) if logits else None)
-        status = fused_project(flat, weight, _native.EPI_ARGMAX, out, norm_weight, eps, ids=ids, top=top,
-                               config=_as_config(choice), sumsq=sumsq)
+        status = launch(choice, weight, flat, out, ids, top)
     else:
         status = _native.FTK_ERR_UNSUPPORTED if prefer_native(m, config) else \
             fused_project(flat, weight, _native.EPI_ARGMAX, out, norm_weight, eps, residual=res, ids=ids, top=top,
