@@ -448,8 +448,9 @@ static int plan(int64_t M, int64_t N, int64_t K, int epi, int cus, const ftk_con
     int rows = cfg && cfg->rows_per_wave ? cfg->rows_per_wave : d.rows;
     // Four rows per tile where the default would leave more than half the CUs
     // without a tile (the shard's QKV at M = 5: 4-row tiles 6.55 us, 8-row 7.08).
-    if (!(cfg && cfg->rows_per_wave) && gemv_tiles(epi, (int)N, rows, kw) < cus / 2 &&
-        quad_supported((int)M, 4, (int)K, kw, epi, pro))
+    // (Only a supported launch has tiles to count: sizes without a default leave rows and kw zero.)
+    if (!(cfg && cfg->rows_per_wave) && quad_supported((int)M, rows, (int)K, kw, epi, pro) &&
+        quad_supported((int)M, 4, (int)K, kw, epi, pro) && gemv_tiles(epi, (int)N, rows, kw) < cus / 2)
       rows = 4;
     const int c = quad_segments((int)K, kw);
     if (c == 0) return FTK_ERR_UNSUPPORTED;  // K is not 128 C KW
