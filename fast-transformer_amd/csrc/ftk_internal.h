@@ -78,15 +78,10 @@ __device__ __forceinline__ u32x2_t out_add4(const ProjArgs& a, int m, int n0) {
   return v;
 }
 
-// One residual element loaded ahead of its use (add_bits): an unconditional load, from x where there
-// is no residual, since a branch around a load ends in a join that waits for it.
-__device__ __forceinline__ uint32_t out_add1(const ProjArgs& a, int m, int n) {
-  const uint16_t* r = a.out_add != nullptr ? a.out_add + (size_t)m * a.N + n : a.x;
-  return *r;
-}
-__device__ __forceinline__ uint32_t add_bits(const ProjArgs& a, float s, uint32_t add) {
-  const uint32_t b = f32_to_bf16(s);
-  return a.out_add == nullptr ? b : f32_to_bf16(bf16_to_f32(b) + bf16_to_f32(add));
+// store_bits with the residual element loaded ahead of its use, in a build whose calls all have a residual:
+// a branch around a load ends in a join that waits for it.
+__device__ __forceinline__ uint32_t add_bits(float s, uint32_t add) {
+  return f32_to_bf16(bf16_to_f32(f32_to_bf16(s)) + bf16_to_f32(add));
 }
 
 // store_bits of four outputs whose residual elements were loaded by out_add4.

@@ -156,7 +156,7 @@ __device__ __forceinline__ void static_for(F&& f) {
 
 }  // namespace
 
-template <int C, int KW, int D, int NX, bool PRO, int EPI, int RT, bool TAIL = false>
+template <int C, int KW, int D, int NX, bool PRO, int EPI, int RT, bool TAIL = false, bool ADD = false>
 __global__ __launch_bounds__(64 * KW) void ring_kernel(ProjArgs a, int tiles) {
   static_assert(C % D == 0, "a tile's units must fill the ring exactly");
   static_assert(NX == 2 || NX == 4, "x rows per unit: 8 or 16");
@@ -279,11 +279,12 @@ __global__ __launch_bounds__(64 * KW) void ring_kernel(ProjArgs a, int tiles) {
   };
 
   // The residual elements of this thread's outputs in the first epilogue, ahead of the units: loaded
-  // where they were added they took four dependent round trips at the end of the walk (three
-  // Qwen3-8B layers at M = 5, the add in O and down: 207.6 us then, 205.8 now).
-  constexpr bool kAdd = EPI == EPI_STORE && !PRO;
+  // where they were added they took four dependent round trips at the end of the walk (4096
+  // outputs at M = 5 / 16, us: O 4096 x 4096 8.2 / 9.2 then, 7.9 / 8.7 now, down 4096 x 12288 18.4 / 21.3
+  // and 18.1 / 21.0). A build of its own (ADD), which plain calls do not pay for.
+  static_assert(!ADD || (EPI == EPI_STORE && !PRO), "the residual add has no norm prologue");
   u32x2_t add0 = {0u, 0u};
-  if constexpr (kAdd) {
+  if constexpr (ADD) {
     const int ln = tid & 63, sub = (tid >> 6) % SUB, i = tid / (64 * SUB);
     const int t = i < my_tiles ? tile_at(i) : 0;
     add0 = out_add4(a, min(ln & 15, M - 1), t * RT + 16 * sub + 4 * (ln >> 4));
@@ -422,14 +423,19 @@ __global__ __launch_bounds__(64 * KW) void ring_kernel(ProjArgs a, int tiles) {
         const int tl = flush_tile(done + i);
         const int n0 = tl * RT + 16 * sub + 4 * gg;
         u32x2_t add = add0;
-        if constexpr (kAdd) {
+        if constexpr (ADD) {
           if (done != 0 || e >= 64 * KW) add = out_add4(a, ll, n0);
         }
         f32x4_t s = part[i][0][sub][ln];
 #pragma unroll
         for (int w = 1; w < KW; ++w) s += part[i][w][sub][ln];
         uint32_t bits[4];
-        store_bits4(a, s, add, bits);
+        if constexpr (ADD) {
+          store_bits4(a, s, add, bits);
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) bits[r] = f32_to_bf16(s[r]);
+        }
         if (a.y != nullptr) store_row4(a.y + (size_t)ll * a.N, n0, a.N, bits);
         if constexpr (EPI == EPI_STORE && RT == 16) {
           if (a.sumsq_out != nullptr) {  // the entry's sum of squares waits in the slot it came from
@@ -700,9 +706,9 @@ static RingKernel pick_ring_tail(int c, int kw, int d, int nx, int rt, bool pro,
 // or three (three only for 8 x rows: 16 would not fit the LDS). NX = 2 serves
 // 2..8 rows, NX = 4 9..16.
 #define FTK_RING_SHAPE(C_, KW_, D_, NX_, RT_, PRO, EPI) \
-  if (c == C_ && kw == KW_ && d == D_ && nx == NX_ && rt == RT_) return ring_kernel<C_, KW_, D_, NX_, PRO, EPI, RT_>;
+  if (c == C_ && kw == KW_ && d == D_ && nx == NX_ && rt == RT_) return ring_kernel<C_, KW_, D_, NX_, PRO, EPI, RT_, false, ADD>;
 
-template <bool PRO, int EPI>
+template <bool PRO, int EPI, bool ADD = false>
 static RingKernel pick_ring_shape(int c, int kw, int d, int nx, int rt) {
   FTK_RING_SHAPE(4, 8, 2, 2, 16, PRO, EPI)
   FTK_RING_SHAPE(4, 8, 2, 4, 16, PRO, EPI)
@@ -720,7 +726,8 @@ static RingKernel pick_ring_shape(int c, int kw, int d, int nx, int rt) {
 }
 #undef FTK_RING_SHAPE
 
-static RingKernel pick_ring(int c, int kw, int d, int nx, int rt, bool pro, int epi) {
+static RingKernel pick_ring(int c, int kw, int d, int nx, int rt, bool pro, int epi, bool add) {
+  if (add) return epi == EPI_STORE && !pro ? pick_ring_shape<false, EPI_STORE, true>(c, kw, d, nx, rt) : nullptr;
   switch (epi) {
     case EPI_STORE: return pro ? pick_ring_shape<true, EPI_STORE>(c, kw, d, nx, rt)
                                : pick_ring_shape<false, EPI_STORE>(c, kw, d, nx, rt);
@@ -735,7 +742,7 @@ static RingKernel pick_ring(int c, int kw, int d, int nx, int rt, bool pro, int 
 bool ring_supported(int M, int K, int kw, int depth, int epi, bool pro, int rows) {
   const int c = quad_segments(K, kw);
   return M >= 1 && M <= kRingMaxRows && c > 0 &&
-         pick_ring(c, kw, depth, ring_x_loads(M), rows, pro, epi) != nullptr;
+         pick_ring(c, kw, depth, ring_x_loads(M), rows, pro, epi, false) != nullptr;
 }
 
 bool ring_tail_supported(int M, int K, int kw, int depth, int epi, bool pro, int rows) {
@@ -749,7 +756,8 @@ hipError_t launch_ring(const ProjArgs& a, int epi, const RingShape& sh, hipStrea
   RingKernel k = nullptr;
   if (c > 0 && a.claim != nullptr)
     k = pick_ring_tail(c, sh.kw, sh.depth, ring_x_loads(a.M), sh.rows, a.gamma != nullptr, epi);
-  if (k == nullptr && c > 0) k = pick_ring(c, sh.kw, sh.depth, ring_x_loads(a.M), sh.rows, a.gamma != nullptr, epi);
+  if (k == nullptr && c > 0)
+    k = pick_ring(c, sh.kw, sh.depth, ring_x_loads(a.M), sh.rows, a.gamma != nullptr, epi, a.out_add != nullptr);
   if (k == nullptr || a.M < 1 || a.M > kRingMaxRows) return hipErrorInvalidValue;
   if (sh.grid < 1 || sh.grid > sh.tiles) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k, dim3(sh.grid), dim3(64 * sh.kw), 0, stream, a, sh.tiles);

@@ -35,8 +35,9 @@
 namespace ftk {
 
 // MR: rows the kernel is built for; a.M <= MR rows are real (the rest are zero
-// and never stored). W: waves per workgroup (4, or 8 when KW = 8).
-template <int MR, int RPW, int C, int KW, int W, bool PRO, int EPI>
+// and never stored). W: waves per workgroup (4, or 8 when KW = 8). ADD: the outputs
+// join a residual (a.out_add).
+template <int MR, int RPW, int C, int KW, int W, bool PRO, int EPI, bool ADD>
 __global__ __launch_bounds__(64 * W) void stream_kernel(ProjArgs a, int tiles) {
   constexpr int T = 64 * W;
   constexpr int GROUPS = W / KW;
@@ -115,15 +116,17 @@ __global__ __launch_bounds__(64 * W) void stream_kernel(ProjArgs a, int tiles) {
   // The residual elements of this thread's first output (of the walk, or of the tile where a wave
   // stores its own: lane p holds slot p's), ahead of the weights. Loaded where they are added, after
   // the last sum, they cost a memory round trip: the 28 layers of Qwen3-0.6B at M = 1, two such
-  // launches each, take 385.7 us with this against 391.0; the 8B layers the same either way.
-  constexpr bool kAdd = EPI == EPI_STORE && !PRO;
-  uint32_t add[kAdd ? MR : 1];
+  // launches each, take 385.7 us with this against 391.0; the 8B layers the same either way. A build
+  // of its own: with the loads' registers and addresses in it, plain calls took longer (3 rows of
+  // 6144 x 1024 4.9 -> 5.4 us, of 4096 x 4096 8.2 -> 8.5).
+  static_assert(!ADD || (EPI == EPI_STORE && !PRO), "the residual add has no norm prologue");
+  uint32_t add[ADD ? MR : 1];
   auto load_add = [&](int t, int g, int p) {
     const int col = gemv_output(t, g, p, PW, GROUPS);
 #pragma unroll
-    for (int m = 0; m < MR; ++m) add[m] = out_add1(a, m < M ? m : 0, col < outputs ? col : outputs - 1);
+    for (int m = 0; m < MR; ++m) add[m] = a.out_add[(size_t)(m < M ? m : 0) * a.N + (col < outputs ? col : outputs - 1)];
   };
-  if constexpr (kAdd) {
+  if constexpr (ADD) {
     if constexpr (KW == 1) {
       load_add(tile, grp, lane % PW);
     } else {
@@ -255,10 +258,10 @@ __global__ __launch_bounds__(64 * W) void stream_kernel(ProjArgs a, int tiles) {
 #pragma unroll
         for (int m = 0; m < MR; ++m) {
           const float s = wave_sum(acc[p][m]);
-          if constexpr (kAdd) {
-            if (lane == p && m < M && col < outputs) a.y[(size_t)m * a.N + col] = (uint16_t)add_bits(a, s, add[m]);
+          if constexpr (ADD) {
+            if (lane == p && m < M && col < outputs) a.y[(size_t)m * a.N + col] = (uint16_t)add_bits(s, add[m]);
           } else if constexpr (EPI == EPI_STORE) {
-            if (lane == 0 && m < M && col < outputs) a.y[(size_t)m * a.N + col] = (uint16_t)store_bits(a, s, m, col);
+            if (lane == 0 && m < M && col < outputs) a.y[(size_t)m * a.N + col] = (uint16_t)f32_to_bf16(s);
           } else {
             const float u = wave_sum(acc[PW + p][m]);
             if (lane == 0 && m < M && col < outputs) a.y[(size_t)m * (a.N / 2) + col] = (uint16_t)swiglu_bf16(s, u);
@@ -277,7 +280,7 @@ __global__ __launch_bounds__(64 * W) void stream_kernel(ProjArgs a, int tiles) {
     ++count;
     if (next >= tiles) break;
     tile = next;
-    if constexpr (kAdd && KW == 1) load_add(tile, grp, lane % PW);
+    if constexpr (ADD && KW == 1) load_add(tile, grp, lane % PW);
   }
   if constexpr (KW == 1 && EPI != EPI_ARGMAX) return;  // every output is stored
   __syncthreads();
@@ -303,10 +306,10 @@ __global__ __launch_bounds__(64 * W) void stream_kernel(ProjArgs a, int tiles) {
       float s = part[i][g * KW][p][m];
 #pragma unroll
       for (int k = 1; k < KW; ++k) s += part[i][g * KW + k][p][m];
-      if constexpr (kAdd) {
-        a.y[(size_t)m * a.N + col] = (uint16_t)(e < T ? add_bits(a, s, add[m]) : store_bits(a, s, m, col));
+      if constexpr (ADD) {
+        a.y[(size_t)m * a.N + col] = (uint16_t)(e < T ? add_bits(s, add[m]) : store_bits(a, s, m, col));
       } else if constexpr (EPI == EPI_STORE) {
-        a.y[(size_t)m * a.N + col] = (uint16_t)store_bits(a, s, m, col);
+        a.y[(size_t)m * a.N + col] = (uint16_t)f32_to_bf16(s);
       } else if constexpr (EPI == EPI_SWIGLU) {
         float u = part[i][g * KW][PW + p][m];
 #pragma unroll
@@ -391,9 +394,9 @@ typedef void (*StreamKernel)(ProjArgs, int);
   FTK_STREAM_SHAPE(1, 1, 8, 1, PRO, EPI)
 
 #define FTK_STREAM_SHAPE(MR, R, CC, KW, PRO, EPI) \
-  if (rpw == R && c == CC && kw == KW) return stream_kernel<MR, R, CC, KW, (KW > kWaves ? KW : kWaves), PRO, EPI>;
+  if (rpw == R && c == CC && kw == KW) return stream_kernel<MR, R, CC, KW, (KW > kWaves ? KW : kWaves), PRO, EPI, ADD>;
 
-template <int MR, bool PRO, int EPI>
+template <int MR, bool PRO, int EPI, bool ADD = false>
 static StreamKernel pick_stream_shape(int rpw, int c, int kw) {
   if constexpr (MR == kStreamMaxRows) {
     FTK_STREAM_SHAPES_8(PRO, EPI)
@@ -411,7 +414,8 @@ static StreamKernel pick_stream_shape(int rpw, int c, int kw) {
 #undef FTK_STREAM_SHAPE
 
 template <int MR>
-static StreamKernel pick_stream_mr(int rpw, int c, int kw, bool pro, int epi) {
+static StreamKernel pick_stream_mr(int rpw, int c, int kw, bool pro, int epi, bool add) {
+  if (add) return epi == EPI_STORE && !pro ? pick_stream_shape<MR, false, EPI_STORE, true>(rpw, c, kw) : nullptr;
   switch (epi) {
     case EPI_STORE: return pro ? pick_stream_shape<MR, true, EPI_STORE>(rpw, c, kw)
                                : pick_stream_shape<MR, false, EPI_STORE>(rpw, c, kw);
@@ -423,28 +427,28 @@ static StreamKernel pick_stream_mr(int rpw, int c, int kw, bool pro, int epi) {
   return nullptr;
 }
 
-static StreamKernel pick_stream(int M, int rpw, int c, int kw, bool pro, int epi) {
+static StreamKernel pick_stream(int M, int rpw, int c, int kw, bool pro, int epi, bool add) {
   switch (M) {
-    case 1: return pick_stream_mr<1>(rpw, c, kw, pro, epi);
-    case 2: return pick_stream_mr<2>(rpw, c, kw, pro, epi);
-    case 3: return pick_stream_mr<3>(rpw, c, kw, pro, epi);
-    case 4: return pick_stream_mr<4>(rpw, c, kw, pro, epi);
+    case 1: return pick_stream_mr<1>(rpw, c, kw, pro, epi, add);
+    case 2: return pick_stream_mr<2>(rpw, c, kw, pro, epi, add);
+    case 3: return pick_stream_mr<3>(rpw, c, kw, pro, epi, add);
+    case 4: return pick_stream_mr<4>(rpw, c, kw, pro, epi, add);
     case 5:
     case 6:
     case 7:
-    case 8: return pick_stream_mr<kStreamMaxRows>(rpw, c, kw, pro, epi);
+    case 8: return pick_stream_mr<kStreamMaxRows>(rpw, c, kw, pro, epi, add);
   }
   return nullptr;
 }
 
 bool stream_supported(int M, int rpw, int K, int kw, int epi) {
   const int c = stream_chunks(K, kw);
-  return c > 0 && pick_stream(M, rpw, c, kw, false, epi) != nullptr;
+  return c > 0 && pick_stream(M, rpw, c, kw, false, epi, false) != nullptr;
 }
 
 hipError_t launch_stream(const ProjArgs& a, int epi, const StreamShape& s, hipStream_t stream) {
   const int c = stream_chunks(a.K, s.kw);
-  StreamKernel k = c > 0 ? pick_stream(a.M, s.rpw, c, s.kw, a.gamma != nullptr, epi) : nullptr;
+  StreamKernel k = c > 0 ? pick_stream(a.M, s.rpw, c, s.kw, a.gamma != nullptr, epi, a.out_add != nullptr) : nullptr;
   if (k == nullptr) return hipErrorInvalidValue;
   // Every workgroup walks at most kStreamMaxTiles tiles (their totals wait in LDS).
   if (s.grid < 1 || s.grid > s.tiles || (s.tiles + s.grid - 1) / s.grid > kStreamMaxTiles)
