@@ -293,32 +293,77 @@ static MfmaLdsDefault mfma_lds_default(int64_t M, int epi, bool pro, int64_t N, 
 constexpr int kMfmaDefaultUnroll = 4;
 constexpr int kMfmaDefaultWaves = 16;
 
-// Where FLOW (a prologue, SwiGLU or argmax) or the MFMA kind's LDS-fed form (a plain STORE) comes
-// before QUAD, STAGE, STREAM and GEMV. us per graph node on MI355X over distinct weights, the kind
-// there otherwise against the one chosen here:
-//   5..16 rows, K without a RING build: norm 4096 x 1024 at M = 8 / 16 QUAD 5.6 / MFMA's registers
-//     7.0 against 5.3 / 5.3; gate/up 6144 x 1024 7.5 / 8.5 against 5.8 / 6.3, 19456 x 2560 30 / 35
-//     against 20 / 19; lm_head 151936 x 1024 184 / 228 against 55 / 55.
-//   2..4 rows: where only GEMV is built (norm 4096 x 2560 at M = 2 / 4 8.2 / 10.8 against 8.3 / 8.4,
-//     gate/up 19456 x 2560 23 / 34 against 20 / 20), lm_head (50257 x 2048 43.8 / 44.6 against 38.4),
-//     and at 3..4 rows gate/up (6144 x 1024 6.0 against 5.8, 12288 x 2048 12.0 against 11.4) and plain
-//     projections of fewer than 16 rows per CU (2048 x 2048 5.0 against 4.2, 1536 x 4096 6.1
-//     against 4.9). Wider plain ones keep the STREAM launches of the 8B shapes.
-//   one row, where only GEMV is built: plain projections (1920 x 5760 9.9 against 6.0, 2560 x 9728 17.6
-//     against 10.7, 5120 x 15360 29.6 against 27.7; K in whole 128-byte lines, as GEMV's loads have no
-//     such need), and FLOW from 8192 outputs (gate/up 19456 x 2560 23.8 against 20.4; norm
-//     4096 x 2560 7.4 against 8.4).
-//   17..32 rows: everything (callers that want the native GEMM there do not come here).
-static bool wide_first(int64_t M, int epi, bool pro, int64_t N, int64_t K, int cus, bool quad, bool stage, bool stream) {
-  const bool plain = !pro && epi == FTK_EPI_STORE;
-  if (!plain && !flow_fits(M, epi, pro, K)) return false;
-  if (M > 4) return !stage && !(M <= 8 && quad && K == 4096);
-  if (M > 1) {
-    if (plain) return !stream || (M >= 3 && N <= 12ll * cus);
-    return !(quad || stream) || (K != 4096 && (epi == FTK_EPI_ARGMAX || (M >= 3 && epi == FTK_EPI_SWIGLU)));
+// Where FLOW (a prologue, SwiGLU or argmax) or the MFMA kind's LDS-fed form (a plain STORE) comes before
+// QUAD, STAGE, STREAM and GEMV. `quad`: QUAD is built and preferred (quad_preferred), `stage`, `stream`: built.
+// All times are us per graph node on MI355X over distinct weights (every kind of every shape timed, K 512 to
+// 16384, 256 to 32768 rows), the kind there otherwise against FLOW or the tiles. From 17 rows everything comes
+// here (callers that want the native GEMM do not).
+//
+// Plain projections: the LDS-fed tiles.
+//   5..16 rows: wherever STAGE is not built.
+//   3..4 rows beside STREAM: of fewer than 12 outputs per CU (2048 x 2048 at 4 rows 4.5 / 4.1), but not so few
+//     that the tiles leave most CUs idle (at 3 rows 1024 x 2048 3.4 / 3.6).
+//   Beside GEMV (any other K): a GEMV whose waves split K (gemv_default) leads for few outputs (one row 512 x
+//     6144 4.1 / 4.8, 2048 x 6144 7.1 / 6.7; two rows 512 x 5120 4.3 / 4.6, 768 x 5120 4.9 / 4.7), any other
+//     nowhere (3072 x 9728 16.9 / 13.1), except at one row in one round of 24-row tiles of K to 5632 (6144 x
+//     2560 7.6 / 8.1). Rows a multiple of 4 KB apart, taken 16 or 24 at once, meet in the same memory channels,
+//     and a GEMV's single rows do not: 8192 x 8192 26.1 / 29.5 at one row, 26.0 / 28.8 at two, 6144 x 10240
+//     23.0 / 25.4 at one (K = 16384: 8 rows too, 2048 outputs 14.8 / 16.8 at one row).
+static bool tiles_first(int64_t M, int64_t N, int64_t K, int cus, bool stage, bool stream) {
+  if (M > 4) return !stage;
+  if (stream) return M >= 3 && N <= 12ll * cus && (N > 2 * (5 - M) * cus || (M == 4 && K <= 1024));
+  if (M > 2) return true;
+  const bool split = gemv_default(FTK_EPI_STORE, N, K).kw > 1;
+  if (split && (N <= (M == 1 ? 4ll : 2ll) * cus || (M == 1 && K > 14336))) return false;
+  const int rows = mfma_lds_default(M, FTK_EPI_STORE, false, N, K, cus).rows;
+  if (M == 2) return !(rows == 16 && K % 8192 == 0);
+  if (rows == 16 && K % 2048 == 0) return false;
+  if (rows == 24 && ((K > 1152 && K <= 5632) || (K % 2048 == 0 && K <= 14336))) return false;
+  return K % 64 == 0;  // whole 128-byte lines, as GEMV's loads have no such need
+}
+
+// Every other projection: FLOW, whose workgroups each load, sum and normalise x before their first product,
+// so it needs tiles enough for that.
+//   5..8 rows beside QUAD (the norm, STORE): more tiles than half the CUs (at 5 rows 2048 x 2048 5.3 / 6.2,
+//     12288 x 2048 13.7 / 11.5, 3072 x 1024 5.1 / 4.9), at up to 6 rows and K past 1024 more tiles than CUs
+//     (4096 x 3072 8.9 / 9.3).
+//   2..4 rows beside QUAD: gate/up from 1.5 tiles per CU and 1024 of K (4 rows 6144 x 1024 6.1 / 5.9, 4096 x
+//     2048 6.7 / 7.3, 12288 x 2048 12.6 / 12.1, 6144 x 3072 10.9 / 11.0), at K = 1024 to 6 per CU (24576 x
+//     1024 13.3 / 12.5, 27648 13.8 / 14.7), without the norm past half the CUs (3 rows 2048 x 3072 5.2 / 5.5,
+//     3072 x 3072 7.1 / 6.1); vocabularies without the norm at any size (3 rows 8000 x 2048 12.7 / 11.1),
+//     with it from a tile per CU and 1024 of K (8000 x 2048 12.1 / 13.0, 18992 x 2048 23.1 / 19.5). At a K that
+//     RING is built for (4096) QUAD stays: with the norm FLOW is 0.74 to 1.03 times as fast.
+//   2..4 rows beside GEMV: nearly everywhere (19456 x 2560 at 2 / 4 rows 23.8 / 21.0, 34.5 / 20.9; norm 2048 x
+//     2560 at 4 rows 9.9 / 7.4). Not the few tiles of a GEMV whose waves split K (norm, 1024 x 5120 at 2 / 3
+//     rows 7.2 / 10.1, 9.3 / 10.2), nor with the norm two ranges of K at two rows: 1024..2048 with one to 2.5
+//     tiles per CU (gate/up 6144 x 1600 7.9 / 8.4) and 3072..4096 with at most one (4096 x 3584 10.6 / 11.4).
+//   One row, where only GEMV is built: from more than two tiles per CU (norm 8192 x 2560 10.4 / 11.4, 9216
+//     14.7 / 12.4; gate/up 9216 x 2560 14.5 / 12.9, 19456 23.4 / 20.8).
+static bool flow_first(int64_t M, int epi, bool pro, int64_t N, int64_t K, int cus, bool quad, bool stage, bool stream) {
+  if (!flow_fits(M, epi, pro, K)) return false;
+  const int64_t tiles = flow_tiles(epi, (int)N, 16);
+  if (M > 4) {
+    if (stage) return false;
+    return !quad || tiles > (M <= 6 && K > 1024 ? cus : cus / 2);
+  }
+  if (M == 1) return !stream && tiles > 2ll * cus;
+  if (quad) {
+    if (ring_supported((int)M, (int)K, 8, 2, epi, pro, 16)) return false;
+    if (epi == FTK_EPI_ARGMAX) return !pro || tiles * 1024 >= cus * K;
+    if (epi == FTK_EPI_SWIGLU && !pro) return tiles > cus / 2;
+    return epi == FTK_EPI_SWIGLU && 2 * tiles * 1024 >= 3 * cus * K && (tiles <= 6ll * cus || K > 1024);
   }
   if (stream) return false;
-  return plain ? K % 64 == 0 : gemv_outputs(epi, (int)N) >= 8192;
+  if (epi == FTK_EPI_ARGMAX) return true;
+  if (gemv_default(epi, N, K).kw > 1) return tiles > (epi == FTK_EPI_SWIGLU && pro ? 2 * cus : cus) >> (M - 1);
+  if (M > 2 || !pro) return true;
+  if (K > 1024 && K < 2048) return tiles <= cus || 2 * tiles > 5ll * cus;
+  return !(K > 3072 && K < 4096 && tiles <= cus);
+}
+
+static bool wide_first(int64_t M, int epi, bool pro, int64_t N, int64_t K, int cus, bool quad, bool stage, bool stream) {
+  return !pro && epi == FTK_EPI_STORE ? tiles_first(M, N, K, cus, stage, stream)
+                                      : flow_first(M, epi, pro, N, K, cus, quad, stage, stream);
 }
 
 static int64_t argmax_keys_bytes(int grid, int64_t M) { return kWsKeys + (int64_t)grid * M * 8; }
