@@ -14,7 +14,7 @@
 // arithmetic (they may hold NaN).
 //
 // Two kernels: the tile kernel (ftk_attn_tile.hip, any shape) and QUAD below
-// (D = 128, up to 4 heads per KV head, short intervals); launch_attention holds the rule.
+// (D = 128, up to 4 heads per KV head); the planner's attn_quad_first holds the rule.
 #include "../../include/ftk.h"
 #include "ftk_attn.h"
 #include "ftk_internal.h"
@@ -417,12 +417,7 @@ hipError_t launch_attention(const AttnArgs& a, const AttnShape& s, hipStream_t s
   while ((1 << log) < s.splits) ++log;
   args.split_magic = (uint32_t)(((uint64_t)1 << (31 + log)) / s.splits + 1);
   args.split_shift = 31 + log;
-  // A wave with at most one 32-slot unit even at a full cache has nothing to pipeline, and the way through
-  // LDS is then pure latency: QUAD keeps those (QKV rows, 8 KV heads x 4: B = 1 x 4K slots in 128-slot
-  // intervals 10.9 us against 11.7, 1K in 64-slot intervals 9.1 against 9.6). From two units on the tile
-  // kernel leads (256-slot intervals 12.0 against 12.9, 512-slot ones 14.0 against 16.5).
-  const bool quad = s.kind == FTK_ATTN_QUAD && s.chunk <= kTileSlots * s.waves;
-  hipError_t e = !quad                 ? launch_attn_tile(args, s, stream)
+  hipError_t e = !s.quad               ? launch_attn_tile(args, s, stream)
                  : a.packed != nullptr ? launch_quad<true>(args, s, stream)
                                        : launch_quad<false>(args, s, stream);
   if (e != hipSuccess || s.splits == 1) return e;

@@ -105,8 +105,10 @@ __device__ __forceinline__ float low_part(float p) {
 // that slot's key and value from the packed row too: it writes them to the cache, reads only the
 // slots before it from memory, and starts wave 0's softmax state with the new slot (score s, p = 1).
 // No other workgroup of the launch reads that slot.
+// (Two waves per SIMD, which the LDS allows at most: without that bound the four-wave builds kept part of
+// their state in accumulation registers and moved it back and forth, 1 to 2 % of every call.)
 template <int D, int W, bool ROPE>
-__global__ __launch_bounds__(64 * W) void attn_tile_kernel(AttnArgs a) {
+__global__ __launch_bounds__(64 * W, 2) void attn_tile_kernel(AttnArgs a) {
   constexpr int CH = D / 8;              // 16-byte chunks per cache row
   constexpr int S = D / 32, DT = D / 16;  // MFMA steps of a score, dimension tiles of the numerator
   constexpr int SLOTS = kTileSlots;      // a unit: 32 cache rows of K and of V

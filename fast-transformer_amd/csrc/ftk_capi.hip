@@ -676,6 +676,26 @@ static bool attn_one_interval(int64_t B, int64_t C, int64_t D, int64_t splits) {
   return C <= kAttnOneInterval || (C <= kAttnOneIntervalWide && (D == 64 || splits <= 2));
 }
 
+// QUAD's own kernel, where its kind is planned or asked for, else the tile kernel. All in us, QUAD against the
+// tile kernel, 8 KV heads, full cache / a tenth of it:
+//   A wave with at most one 32-slot unit even at a full cache has nothing to pipeline, and the way through LDS is
+//   then pure latency: 1 x 4K slots in 128-slot intervals 10.8 / 9.1 against 11.6 / 9.4, 1K in 64-slot ones 8.8 /
+//   8.6 against 9.4 / 8.9.
+//   One row: two units per wave (1 x 8K in 256-slot intervals 13.4 / 9.0 against 13.7 / 9.6), and with one or two
+//   heads per KV head, for which the tile kernel fills an eighth of its columns or a quarter, at any length (one
+//   head 1 x 8K 12.5 / 8.8 against 13.5 / 9.4, 1 x 32K 28.1 / 11.0 against 28.8 / 12.3; 4 heads there 29.9 / 11.7
+//   against 29.1 / 13.1).
+//   Several rows with one or two heads: two units per wave, in several intervals (one head 4 x 2K 12.2 / 8.0
+//   against 13.3 / 9.1) or where the rows fill the CUs (one head 32 x 256 9.7 / 6.0 against 10.6 / 6.6). Rows at
+//   different places of their caches gain most from the tile kernel (4 heads, positions spread over 10..100 %: 4 x
+//   2K 12.7 against 12.0, 4 x 8K 28.7 against 23.5), so everything else is its.
+static bool attn_quad_first(int64_t B, int64_t G, int groups, int64_t splits, int64_t chunk, int waves, int cus) {
+  const int64_t unit = 32ll * waves;  // a tile step of every wave
+  if (chunk <= unit) return true;
+  if (B == 1 && splits > 1) return G <= 2 || chunk <= 2 * unit;
+  return G <= 2 && chunk <= 2 * unit && (splits > 1 || groups >= cus);
+}
+
 static int attn_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t C, int64_t D, int cus, const ftk_attn_config* cfg,
                      ftk_attn_plan* p, AttnShape* shape) {
   if (B < 1 || Hq < 1 || Hkv < 1 || C < 1 || Hq % Hkv || cus < 1) return FTK_ERR_INVALID;
@@ -722,7 +742,10 @@ static int attn_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t C, int64_t D, i
   p->unroll = unroll;
   p->grid = (int)(groups * splits);
   p->workspace_bytes = splits > 1 ? (int64_t)groups * splits * G * (D + 2) * 4 : 0;
-  if (shape) *shape = AttnShape{kind, (int)D, (int)G, groups, (int)splits, (int)chunk, waves, unroll};
+  if (shape) {
+    const bool quad = kind == FTK_ATTN_QUAD && attn_quad_first(B, G, groups, splits, chunk, waves, cus);
+    *shape = AttnShape{kind, (int)D, (int)G, groups, (int)splits, (int)chunk, waves, unroll, quad};
+  }
   return FTK_OK;
 }
 

@@ -403,6 +403,7 @@ struct AttnShape {
   int chunk;       // slots per interval at a full cache
   int waves;       // W: waves per workgroup (4, 8)
   int unroll;      // QUAD: groups of 16 cache rows per wave step (1, 2)
+  bool quad;       // the QUAD kernel (attn_quad_first), else the tile kernel
 };
 constexpr int kAttnMaxGroup = 8;
 constexpr int kAttnMaxSplits = 1024;  // slot intervals per group the merge kernel takes
