@@ -652,14 +652,15 @@ static int64_t call_workspace(const ftk_plan& p, int epi, bool pro) {
 
 // ---- decode attention: launch planning --------------------------------------
 
-// Workgroups the default split count aims at: one per CU (measured on MI355X:
-// 32 intervals per KV head beat 64 at B = 1 from 1K to 32K slots).
+// Workgroups the default split count aims at: one per CU (one row, 8 KV heads x 4 on MI355X, 32 intervals
+// against 64: full 16K 18.9 / 19.2 us, 32K 29.1 / 29.2, 64K 48.2 / 48.8; half full 32K 20.3 / 19.6).
 constexpr int kAttnGroupsPerCu = 1;
 // Several rows over caches of more than 4K slots: intervals of 1K slots, up to four workgroups per CU, so
 // that rows standing at different places of their caches even out (8 KV heads x 4, positions spread over
-// 10%..100% of the cache: 16 x 8K 73.5 -> 57.4 us with 8 intervals instead of 2, 64.8 with 2; 32 x 8K 133 ->
-// 105; 4 x 16K 42 -> 34; 512-slot intervals and shorter lose again, 4 x 16K 35). At 4K slots the extra
-// intervals gain under 1% (16 rows: 51.4 -> 51.0 us).
+// 10%..100% of the cache, intervals for one / two / four workgroups per CU: 16 x 8K 59.6 / 54.6 / 52.7 us, 8 x
+// 16K 62.5 / 55.7 / 52.1; 4 x 8K in 1K-slot intervals 22.7, in 512-slot ones 20.1, 256-slot 23.6). Rows that all
+// stand early pay for it (a tenth full 16 x 8K 17.6 / 16.7 / 22.0, 32 x 8K 22.1 / 24.9 / 27.2; spread the
+// latter takes 105.3 / 100.5 / 99.7).
 constexpr int kAttnGroupsPerCuLong = 4;
 constexpr int64_t kAttnLongSlots = 4096, kAttnLongChunk = 1024;
 
