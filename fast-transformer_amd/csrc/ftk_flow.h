@@ -218,20 +218,24 @@ __global__ __launch_bounds__(512) void flow_kernel(ProjArgs a, int tiles) {
   for (int f = 0; f < OV; ++f)
     if (wf < F) issue_w();
 
-  // A ragged last segment: nothing past K.
+  // A ragged last segment: nothing past K, for the norm's sums and, as the gain read there may be infinite,
+  // once more after it.
   const int tail = (K & 127) && (segs - 1) % KW == kw ? (segs - 1) / KW : -1;  // its unit, or -1
-  unroll_for<0, CM>([&](auto J) {
-    constexpr int j = decltype(J)::value;
-    if (j == tail) {
-      const u32x4_t zero = {0u, 0u, 0u, 0u};
+  auto clear_tail = [&]() {
+    unroll_for<0, CM>([&](auto J) {
+      constexpr int j = decltype(J)::value;
+      if (j == tail) {
+        const u32x4_t zero = {0u, 0u, 0u, 0u};
 #pragma unroll
-      for (int s = 0; s < 4; ++s)
-        if ((j * KW + kw) * 128 + 32 * s + 8 * g >= K) {
+        for (int s = 0; s < 4; ++s)
+          if ((j * KW + kw) * 128 + 32 * s + 8 * g >= K) {
 #pragma unroll
-          for (int m = 0; m < MB; ++m) xr[j][m][s] = zero;
-        }
-    }
-  });
+            for (int m = 0; m < MB; ++m) xr[j][m][s] = zero;
+          }
+      }
+    });
+  };
+  clear_tail();
 
   // ---- RMSNorm: the rows' sums of squares from the operands, then the operands normalised in place
   if constexpr (PRO) {
@@ -265,6 +269,7 @@ __global__ __launch_bounds__(512) void flow_kernel(ProjArgs a, int tiles) {
 #pragma unroll
         for (int s = 0; s < 4; ++s) xr[j][m][s] = norm8(xr[j][m][s], gn[s], scale[m]);
     });
+    clear_tail();
   }
 
   // ---- epilogue of the parked tiles done .. done + count - 1: thread e takes (tile, column block, lane position);
