@@ -662,7 +662,8 @@ def _linear(x, weight, sumsq):
             return project(inp, w, _as_config(choice))
 
         choice = _choice("linear", flat, weight, run, lambda w, inp=flat: F.linear(inp, w))
-    if choice == "native":
+    # (Unaligned rows or weights have the scalar kernel here: from 17 rows the native GEMM, as ever.)
+    if choice == "native" or (choice is None and prefer_native(rows) and not _fusable(flat, weight)):
         return F.linear(x, weight)
     out = project(flat, weight, _as_config(choice), sumsq=sumsq)
     return out if x.dim() == 2 else out.reshape(*x.shape[:-1], weight.shape[0])
