@@ -395,7 +395,8 @@ static hipError_t launch_quad(const AttnArgs& a, const AttnShape& s, hipStream_t
   }
 }
 
-// Which configurations of the ROWS kind a caller may name (heads per group and cache rows in flight).
+// Which `unroll` of the ROWS kind a caller may name for g heads per group: what the interface has always taken
+// (the kernel is the same for all of them; they size the default intervals).
 constexpr bool attn_fits(int g, int u) { return 24 + 18 * u + 17 * g + g * u <= 230; }
 
 bool attn_supported(int kind, int dim, int group_size, int waves, int unroll) {

@@ -255,7 +255,7 @@ static bool ring_preferred(int64_t M, int epi, bool pro, int64_t N, int64_t K, i
 // FLOW: every projection with a prologue, SwiGLU and argmax whose x rows fit its registers.
 static bool flow_fits(int64_t M, int epi, bool pro, int64_t K) {
   return K % 8 == 0 && K <= INT32_MAX && flow_segments((int)K) <= kFlowMaxSegments && M <= kFlowMaxRows &&
-         flow_supported((int)M, (int)K, 16, epi, pro);
+         flow_supported((int)M, (int)K, epi, pro);
 }
 
 // The MFMA kind's LDS-fed form: the fewest rows per tile that give every tile a CU of its own
@@ -341,7 +341,7 @@ static bool tiles_first(int64_t M, int64_t N, int64_t K, int cus, bool stage, bo
 //     14.7 / 12.4; gate/up 9216 x 2560 14.5 / 12.9, 19456 23.4 / 20.8).
 static bool flow_first(int64_t M, int epi, bool pro, int64_t N, int64_t K, int cus, bool quad, bool stage, bool stream) {
   if (!flow_fits(M, epi, pro, K)) return false;
-  const int64_t tiles = flow_tiles(epi, (int)N, 16);
+  const int64_t tiles = flow_tiles(epi, (int)N, kFlowTile);
   if (M > 4) {
     if (stage) return false;
     return !quad || tiles > (M <= 6 && K > 1024 ? cus : cus / 2);
@@ -568,11 +568,11 @@ static int plan(int64_t M, int64_t N, int64_t K, int epi, int cus, const ftk_con
   }
   if (kind == FTK_KIND_FLOW) {
     const int waves = cfg && cfg->waves ? cfg->waves : kFlowWaves;
-    const int rows = cfg && cfg->rows_per_wave ? cfg->rows_per_wave : 16;
+    const int rows = cfg && cfg->rows_per_wave ? cfg->rows_per_wave : kFlowTile;
     if (M > kFlowMaxRows || flow_segments((int)K) > kFlowMaxSegments) return FTK_ERR_UNSUPPORTED;
-    if (waves != kFlowWaves || !flow_supported((int)M, (int)K, rows, epi, pro)) return FTK_ERR_INVALID;
+    if (waves != kFlowWaves || rows != kFlowTile || !flow_supported((int)M, (int)K, epi, pro)) return FTK_ERR_INVALID;
     p->rows_per_wave = rows;
-    p->unroll = flow_depth(rows);
+    p->unroll = kFlowDepth;
     p->waves = waves;
     p->threads = 64 * waves;
     p->tiles = flow_tiles(epi, (int)N, rows);
@@ -714,7 +714,11 @@ static int attn_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t C, int64_t D, i
   if (kind == FTK_ATTN_ROWS && !(cfg && cfg->unroll) && !attn_supported(kind, (int)D, (int)G, waves, unroll))
     unroll = 2;
   if (!attn_supported(kind, (int)D, (int)G, waves, unroll)) return FTK_ERR_INVALID;
-  const int64_t unit = kind == FTK_ATTN_QUAD ? 16 * unroll : (64 / (D / 8)) * unroll;  // slots per wave step
+  // The fewest slots of a default interval, per wave: QUAD's step; for ROWS what `unroll` says, which its kernel,
+  // whose step is 32 slots, does not read. Less than a step per wave is no loss: a short cache is waited for
+  // rather than read (1 x 512 slots, 8 KV heads x 8, us: 16 intervals 8.4, 8 8.5, 4, a step per wave each, 9.1; 1K
+  // slots: 32 intervals 9.1, 8 9.2).
+  const int64_t unit = kind == FTK_ATTN_QUAD ? 16 * unroll : (64 / (D / 8)) * unroll;
   int64_t splits;
   if (cfg && cfg->splits) {
     if (cfg->splits < 1) return FTK_ERR_INVALID;
@@ -728,7 +732,7 @@ static int attn_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t C, int64_t D, i
       const int64_t longer = many < whole ? many : whole;
       if (longer > want) want = longer;
     }
-    const int64_t most = (C + waves * unit - 1) / (waves * unit);  // at least one step per wave
+    const int64_t most = (C + waves * unit - 1) / (waves * unit);
     splits = want < most ? want : most;
     if (splits > kAttnMaxSplits) splits = kAttnMaxSplits;
     if (splits < 1 || attn_one_interval(B, C, D, splits)) splits = 1;
@@ -1092,7 +1096,7 @@ static int project_impl(const void* x, const ftk_rows* rows, const void* gamma, 
     RingShape g = {p.unroll, p.waves, p.grid, p.tiles, p.rows_per_wave};
     e = launch_ring(a, epilogue, g, s);
   } else if (p.kind == FTK_KIND_FLOW) {
-    FlowShape g = {p.rows_per_wave, p.grid, p.tiles};
+    FlowShape g = {p.grid, p.tiles};
     e = launch_flow(a, epilogue, g, s);
   } else if (p.kind == FTK_KIND_GEMV) {
     GemvShape g = {p.rows_per_wave, p.unroll, p.waves, p.grid, p.tiles, (size_t)p.lds_bytes};

@@ -94,19 +94,19 @@ __device__ __forceinline__ void unroll_for(F&& f) {
   }
 }
 
-template <int NX, int CM, int RT, bool PRO, int EPI>
+template <int NX, int CM, bool PRO, int EPI>
 __global__ __launch_bounds__(512) void flow_kernel(ProjArgs a, int tiles) {
-  constexpr int KW = kFlowWaves;
+  constexpr int KW = kFlowWaves, RT = kFlowTile;
   constexpr int MB = (NX + 3) / 4;   // MFMA column blocks of 16 x rows
   constexpr int WL = RT / 4;         // loads per weight unit (4 rows x 256 bytes each)
   constexpr int WS = 16 * RT, XS = 64 * NX;  // 16-byte slots of a weight unit and of an x unit
-  constexpr int D = flow_depth(RT);  // weight units in flight per wave
+  constexpr int D = kFlowDepth;  // weight units in flight per wave
   constexpr int XB = flow_x_batch(NX, CM);   // x units staged at once
-  constexpr int RW = flow_wave_slots(NX, CM, RT);
+  constexpr int RW = flow_wave_slots(NX, CM);
   constexpr int OV = (XB * XS + WS - 1) / WS < D ? (XB * XS + WS - 1) / WS : D;  // ring slots under the staged x
   constexpr int BATCHES = (CM + XB - 1) / XB;
   static_assert(D * WL < 64, "vmcnt is 6 bits");
-  constexpr int DM = flow_parked(NX, CM, RT, PRO);  // tiles parked before an epilogue
+  constexpr int DM = flow_parked(NX, CM, PRO);  // tiles parked before an epilogue
   constexpr int GS = PRO ? 16 * CM : 1;  // gain slots per wave
   __shared__ u32x4_t ring[KW * RW + 256 * MB - XS];  // B operand rows past the loaded ones read on
   __shared__ f32x4_t part[DM][KW][MB][64];
@@ -381,17 +381,16 @@ typedef void (*FlowKernel)(ProjArgs, int);
 template <int NX, int CM, bool PRO>
 FlowKernel pick_flow_epilogue(int epi) {
   switch (epi) {
-    case EPI_STORE: return flow_kernel<NX, CM, 16, PRO, EPI_STORE>;
-    case EPI_SWIGLU: return flow_kernel<NX, CM, 16, PRO, EPI_SWIGLU>;
-    case EPI_ARGMAX: return flow_kernel<NX, CM, 16, PRO, EPI_ARGMAX>;
+    case EPI_STORE: return flow_kernel<NX, CM, PRO, EPI_STORE>;
+    case EPI_SWIGLU: return flow_kernel<NX, CM, PRO, EPI_SWIGLU>;
+    case EPI_ARGMAX: return flow_kernel<NX, CM, PRO, EPI_ARGMAX>;
   }
   return nullptr;
 }
 
 // Kernel for up to 4 NX x rows and CM segments per wave.
 template <int NX, bool PRO>
-FlowKernel pick_flow_segments(int c, int rt, int epi) {
-  if (rt != 16) return nullptr;
+FlowKernel pick_flow_segments(int c, int epi) {
   if (c <= 1) return pick_flow_epilogue<NX, 1, PRO>(epi);
   if (c <= 2) return pick_flow_epilogue<NX, 2, PRO>(epi);
   if (c <= 3) return pick_flow_epilogue<NX, 3, PRO>(epi);

@@ -3,8 +3,8 @@
 
 namespace ftk {
 
-FlowKernel pick_flow_x4(int c, int rt, int epi, bool pro) {
-  return pro ? pick_flow_segments<4, true>(c, rt, epi) : pick_flow_segments<4, false>(c, rt, epi);
+FlowKernel pick_flow_x4(int c, int epi, bool pro) {
+  return pro ? pick_flow_segments<4, true>(c, epi) : pick_flow_segments<4, false>(c, epi);
 }
 
 }  // namespace ftk

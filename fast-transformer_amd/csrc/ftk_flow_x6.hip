@@ -3,8 +3,8 @@
 
 namespace ftk {
 
-FlowKernel pick_flow_x6(int c, int rt, int epi, bool pro) {
-  return pro ? pick_flow_segments<6, true>(c, rt, epi) : pick_flow_segments<6, false>(c, rt, epi);
+FlowKernel pick_flow_x6(int c, int epi, bool pro) {
+  return pro ? pick_flow_segments<6, true>(c, epi) : pick_flow_segments<6, false>(c, epi);
 }
 
 }  // namespace ftk

@@ -343,11 +343,10 @@ hipError_t launch_mfma(const ProjArgs& a, int epi, const MfmaShape& shape, const
 
 // Launch shape of the FLOW kind.
 struct FlowShape {
-  int rows;      // RT: weight rows per tile (8, 12 or 16)
   int grid;      // workgroups; workgroup wg takes tile ring_tile(wg, i, grid, tiles) at step i
   int tiles;
 };
-bool flow_supported(int M, int K, int rt, int epi, bool pro);
+bool flow_supported(int M, int K, int epi, bool pro);
 hipError_t launch_flow(const ProjArgs& a, int epi, const FlowShape& shape, hipStream_t stream);
 
 // Launch shape of the MFMA kind's LDS-fed form (one workgroup per tile).

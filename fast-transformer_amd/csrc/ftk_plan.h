@@ -221,14 +221,16 @@ FTK_HD constexpr int ring_max_depth(int c, int kw, int d, int nx, bool pro, int 
 // ---- M = 1..32 with any K % 8 == 0 up to 5120: the FLOW kind ------------------------
 // A persistent walk as RING's (tile ring_tile(wg, i, G, tiles) at step i), with the
 // K segments dealt to 8 waves (wave kw: kw, kw + 8, ...; the last may be short) and
-// the x rows of a wave's segments in registers throughout. A tile is RT = 8, 12 or 16
-// weight rows, for SwiGLU RT / 2 gate rows and the matching up rows.
+// the x rows of a wave's segments in registers throughout. A tile is 16 weight rows, for
+// SwiGLU 8 gate rows and the matching up rows.
 constexpr int kFlowMaxRows = 32;
+constexpr int kFlowTile = 16;
 constexpr int kFlowWaves = 8;
 constexpr int kFlowMaxSegments = 5;  // per wave
 // Loads of 4 x rows per unit a kernel is built for.
 FTK_HD constexpr int flow_x_loads(int m) { return m <= 4 ? 1 : m <= 8 ? 2 : m <= 16 ? 4 : m <= 24 ? 6 : 8; }
 FTK_HD constexpr int flow_segments(int k) { return ((k + 127) / 128 + kFlowWaves - 1) / kFlowWaves; }
+// Tiles of RT weight rows (SwiGLU: RT / 2 gate and RT / 2 up rows), FLOW's and the LDS-fed MFMA form's.
 FTK_HD constexpr int flow_out_per_tile(int epi, int rt) { return epi == EPI_SWIGLU ? rt / 2 : rt; }
 FTK_HD int flow_tiles(int epi, int n_rows, int rt) {
   const int per = flow_out_per_tile(epi, rt);
@@ -247,16 +249,16 @@ FTK_HD int flow_weight_row(int epi, int t, int r, int n_rows, int rt) {
 }
 // Weight units in flight per wave, x units staged at once (in 16 KiB per wave), and the
 // 16-byte slots of a wave's LDS that hold one or the other.
-FTK_HD constexpr int flow_depth(int rt) { return rt == 16 ? 4 : rt == 12 ? 5 : 8; }
+constexpr int kFlowDepth = 4;
 FTK_HD constexpr int flow_x_batch(int nx, int cm) { return cm * nx <= 16 ? cm : 16 / nx; }
-FTK_HD constexpr int flow_wave_slots(int nx, int cm, int rt) {
-  return flow_depth(rt) * 16 * rt > flow_x_batch(nx, cm) * 64 * nx ? flow_depth(rt) * 16 * rt
-                                                                   : flow_x_batch(nx, cm) * 64 * nx;
+FTK_HD constexpr int flow_wave_slots(int nx, int cm) {
+  return kFlowDepth * 16 * kFlowTile > flow_x_batch(nx, cm) * 64 * nx ? kFlowDepth * 16 * kFlowTile
+                                                                      : flow_x_batch(nx, cm) * 64 * nx;
 }
 // Tiles whose per-wave partials fit beside the rings, the gain and the row sums (at most 4).
-FTK_HD constexpr int flow_parked(int nx, int cm, int rt, bool pro) {
+FTK_HD constexpr int flow_parked(int nx, int cm, bool pro) {
   const int mb = (nx + 3) / 4;
-  const int fixed = (kFlowWaves * flow_wave_slots(nx, cm, rt) + 256 * mb - 64 * nx) * 16 +
+  const int fixed = (kFlowWaves * flow_wave_slots(nx, cm) + 256 * mb - 64 * nx) * 16 +
                     kFlowWaves * (pro ? cm * 256 : 0) + kFlowWaves * 64 * mb + kFlowWaves * 128 + 256;
   const int fit = (160 * 1024 - fixed) / (kFlowWaves * 1024 * mb);
   return fit > 4 ? 4 : fit;

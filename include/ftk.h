@@ -107,7 +107,7 @@ typedef struct ftk_config {
                           (16, 32); QUAD: weight rows per row group per tile (4, 8, 16, 24; SwiGLU
                           8, 16, 24); RING: 16 (SwiGLU: 8 gate + 8 up rows), or for the
                           STORE epilogue 12 (at K = 4096), or 24 (at up to 8 rows);
-                          FLOW: 16, 8 (half of them gate rows for SwiGLU), or 12 (STORE) */
+                          FLOW: 16 (SwiGLU: 8 gate + 8 up rows) */
   int unroll;          /* GEMV: 16-byte chunks per lane per load batch (1, 2, 4);
                           MFMA: K steps of loads in flight per wave (T = 1, 2: 4 or 8; T = 4: 2 or 4), or
                           1: the LDS-fed form (what a zero rows_per_wave, unroll and waves select):
@@ -248,7 +248,8 @@ typedef struct ftk_rows {
 
 /* ftk_project_bf16 with the prologue's rows described by `rows` (NULL: x as is).
  * Needs gamma. Kinds without the fused form return FTK_ERR_UNSUPPORTED (the
- * generic kind; the MFMA kind when sum is NULL). */
+ * generic kind; the MFMA kind's register-fed form when sum is NULL; FLOW and RING
+ * with a residual). */
 int ftk_project_rows_bf16(const void* x, const ftk_rows* rows, const void* gamma, float eps, const void* w, void* y,
                           int64_t M, int64_t N, int64_t K, int epilogue, void* ids, int ids_bytes, float* top,
                           void* workspace, int64_t workspace_bytes, const ftk_config* cfg, void* stream);
@@ -319,13 +320,15 @@ typedef enum ftk_attn_kind {
                          16x16x32 MFMAs, 32 slots of K and V per wave step through LDS */
   FTK_ATTN_QUAD = 2   /* D = 128, up to 4 query heads per KV head: scores on 16-block 4x4x4 MFMAs fed
                          by 4 cache rows x 256 bytes per wave load, one softmax step per (row, head),
-                         p V on the VALU; intervals of more than 32 slots per wave take ROWS' kernel */
+                         p V on the VALU; long intervals take ROWS' kernel (past 32 slots per wave, or
+                         later for one row and for one or two heads per KV head) */
 } ftk_attn_kind;
 typedef struct ftk_attn_config {
   int kind;    /* ftk_attn_kind */
   int splits;  /* slot intervals per (row, KV head), at most 1024; 1 = no merge launch */
   int waves;   /* waves per workgroup (4, 8) */
-  int unroll;  /* ROWS: 2, 4, 8 (8 with up to 2 heads), the same launch; sizes the default split count;
+  int unroll;  /* ROWS: 2, 4 (up to 6 heads), 8 (up to 2 heads): the same kernel, it sizes the default split
+                  count only (intervals of at least waves x unroll x 4 slots, 8 at 64 dimensions);
                   QUAD: groups of 16 cache rows per wave step, the loads of the next step in flight (1, 2) */
 } ftk_attn_config;
 typedef struct ftk_attn_plan {
