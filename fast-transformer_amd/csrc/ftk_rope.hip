@@ -2,8 +2,8 @@
 // step on gfx950: engine/kernels/qk_rope.py:13-94 (_qk_rope_cache).
 //
 // Two forms of one arithmetic: qk_rope_kernel (FP32 partials, or pointers that
-// are not 16-byte aligned) gives one wave to a (row, head); qk_rope_rows_kernel
-// (BF16 rows, 16-byte aligned) gives D / 8 lanes to a head. Arithmetic is FP32
+// are not 16-byte aligned, or few heads of 64) gives one wave to a (row, head);
+// qk_rope_rows_kernel gives D / 8 lanes to a head. Arithmetic is FP32
 // with the reference's roundings: n = bf16(x inv_std), w = bf16(n gain),
 // out = bf16(bf16(w cos) + bf16(rot sin)). Query heads go to the token-major
 // query [rows, Hq, D]; key heads and the copied value heads to the caches
@@ -235,11 +235,17 @@ __global__ __launch_bounds__(kThreads) void qk_rope_rows_kernel(RopeArgs a, int 
 
 namespace {
 
-bool rows_form(const RopeArgs& a) {
+// Few heads of 64 stay with the general form: a launch of a few workgroups is one chain of loads and sums, and
+// with eight elements to a lane it is the longer one. us, general / rows form: 1 x 18 heads 2.1 / 2.3, 32 x 18
+// 2.3 / 2.5, 16 x 80 2.4 / 2.5, 128 x 18 2.5 / 2.6, 64 x 48 2.6 / 2.6, 64 x 80 3.0 / 2.6, 1024 x 80 16.9 / 7.9.
+// Heads of 128 are as fast or faster in the rows form throughout (1 x 6 2.2 / 2.2, 32 x 48 2.5 / 2.5).
+constexpr int64_t kFewHeads64 = 2560;
+
+bool rows_form(const RopeArgs& a, int rows) {
   const void* ptrs[] = {a.packed, a.q_gain, a.k_gain, a.cos, a.sin, a.query, a.keys, a.values};
   for (const void* p : ptrs)
     if (reinterpret_cast<uintptr_t>(p) & 15u) return false;
-  return a.splits == 1;
+  return a.splits == 1 && (a.dim == 128 || (int64_t)rows * (a.q_heads + 2 * a.kv_heads) >= kFewHeads64);
 }
 
 template <int D>
@@ -264,7 +270,7 @@ hipError_t launch_rows(const RopeArgs& a, int rows, hipStream_t stream) {
 }  // namespace
 
 hipError_t launch_qk_rope(const RopeArgs& a, int rows, hipStream_t stream) {
-  if (rows_form(a)) return a.dim == 128 ? launch_rows<128>(a, rows, stream) : launch_rows<64>(a, rows, stream);
+  if (rows_form(a, rows)) return a.dim == 128 ? launch_rows<128>(a, rows, stream) : launch_rows<64>(a, rows, stream);
   constexpr int W = 4;
   const dim3 grid((unsigned)rows, (unsigned)((a.q_heads + a.kv_heads + W - 1) / W));
   if (a.dim == 128)
