@@ -52,11 +52,15 @@ def _both(packed, norms, keys, values, run):
         k, v = keys.clone(), values.clone()
         got.append((run(rows, norms, k, v), k, v))
     (q, k, v), (wq, wk, wv) = got
-    # The two factors of a product may each be a BF16 ulp apart (2^-7), its rounding and the sum's half an
-    # ulp (2^-8): below 2^-5 of |w cos| + |w' sin|, which is at most twice the head's largest output.
+    # n = bf16(x inv_std) may be one BF16 ulp apart (2^-7), w = bf16(n gain) and its product with cos or sin round
+    # twice more each (2^-9 every time): 2^-6 of |w cos| + |w' sin|, which is at most the norm of the pair that is
+    # rotated (cos^2 + sin^2 = 1, to the table's own rounding); the sum's two roundings add 2^-8 of that.
     for a, w in ((q, wq), (k, wk)):
         a, w = a.float(), w.float()
-        assert bool(((a - w).abs() <= 2.0 ** -4 * w.abs().amax(dim=-1, keepdim=True)).all())
+        half = w.shape[-1] // 2
+        pair = torch.hypot(w[..., :half], w[..., half:])
+        pair = torch.cat((pair, pair), dim=-1)
+        assert bool(((a - w).abs() <= 1.02 * (2.0 ** -6 + 2.0 ** -8) * pair).all())
         assert float((a != w).float().mean()) < 2e-3  # inv_std moves by an ulp of FP32: few results round apart
     assert (to_bits(v) == to_bits(wv)).all()
     return got[0]
