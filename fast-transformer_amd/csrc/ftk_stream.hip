@@ -124,7 +124,9 @@ __global__ __launch_bounds__(64 * W) void stream_kernel(ProjArgs a, int tiles) {
   auto load_add = [&](int t, int g, int p) {
     const int col = gemv_output(t, g, p, PW, GROUPS);
 #pragma unroll
-    for (int m = 0; m < MR; ++m) add[m] = a.out_add[(size_t)(m < M ? m : 0) * a.N + (col < outputs ? col : outputs - 1)];
+    for (int m = 0; m < MR; ++m)  // (an atomic load, because a plain one is moved to its use)
+      add[m] = __hip_atomic_load(a.out_add + (size_t)(m < M ? m : 0) * a.N + (col < outputs ? col : outputs - 1),
+                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
   };
   if constexpr (ADD) {
     if constexpr (KW == 1) {
