@@ -3,7 +3,7 @@
 //
 // Long caches are bound by HBM reads, short ones by the chain position -> cache
 // -> softmax -> merge. A wave takes units of 32 cache slots: direct-to-LDS loads
-// bring K and V (64 KB per workgroup at D = 128, two workgroups per CU, no
+// bring K and V (64 KB per workgroup at D = 128, so that two fit a CU, no
 // registers held), the next K is requested as soon as this one's operands are
 // read and the next V as soon as this V's are, so one of the two is in flight
 // throughout. K rows are the A operand and the query heads the B operand's
@@ -17,7 +17,8 @@
 // from 5 heads per KV head on.
 // Measured (partials + merge): 1 x 32K slots, 8 KV heads x 8, 71.1 -> 29.2 us;
 // D = 64 x 4 heads 24.4 -> 16.7; 8 x 2K ragged, 8 heads, 39.4 -> 15.2; 16 x 8K
-// ragged, 4 heads, 72.9 -> 57.3 (8 intervals); 1 x 32K, 4 heads, 28.8 both.
+// ragged, 4 heads, 72.9 -> 57.3 (8 intervals); 1 x 32K, 4 heads, 29.9 -> 29.1
+// (both before and after with the same intervals).
 #include "ftk_attn.h"
 #include "ftk_dma.h"
 

@@ -669,7 +669,8 @@ constexpr int64_t kAttnLongSlots = 4096, kAttnLongChunk = 1024;
 // 4 x 128 7.8 / 6.1, 4 x 256 7.8 / 7.2, 16 x 256 9.4 / 7.7, 8 heads per KV head 1 x 256 6.8 / 5.5, D = 64
 // 4 x 256 6.1 / 4.4. At 320 and 384 slots of 128 dimensions more than two intervals are the faster ones
 // (4 x 384 7.9 / 8.4) and two are not (16 x 384 10.5 / 9.1; D = 64, 4 x 384 6.1 / 5.3). One row of up to
-// 128 slots keeps an interval per step of its waves (its launch is part of the planner's known answers).
+// 128 slots keeps an interval per step of its waves: callers and tests know that launch (1 x 128 x 4 heads in
+// two intervals), and one interval would be the faster one (8.6 / 6.0).
 constexpr int64_t kAttnOneInterval = 256, kAttnOneIntervalWide = 384;
 
 static bool attn_one_interval(int64_t B, int64_t C, int64_t D, int64_t splits) {

@@ -2,7 +2,9 @@
 
 Drop-in for engine/kernels/decode_attention.py:229-258 (``decode_attention``):
 the same signature, shapes, assertions and output layout. BF16 Q/K/V, FP32
-scores and sums, p rounded to BF16 before it weights V, BF16 output. Every
+scores and sums, BF16 output; p weights V as one BF16 value (the QUAD kernel,
+as the reference does) or as two that carry 16 bits of it (the tile kernel).
+An infinite value in a slot the row sees gives that infinity with either. Every
 cache slot up to ``position`` contributes; later slots are never read into
 the result. No host synchronization: the length is read on the device, so a
 captured graph replays for every position.
@@ -11,8 +13,9 @@ Each (row, KV head) pair's slots are cut into intervals ("splits"); a
 workgroup attends to one interval and writes FP32 partials, and a second
 kernel merges them (engine/kernels/decode_attention.py:31-149). With one
 interval the first kernel writes the output itself. The split count is the
-planner's, for MI355X: about two workgroups per CU, at least one load step
-per wave (``ftk_plan_decode_attention``); ``config`` overrides it.
+planner's, for MI355X (``ftk_plan_decode_attention``): one workgroup per CU, up
+to four for several rows over more than 4K slots, one interval for short
+caches; ``config`` overrides it.
 """
 
 import ctypes
@@ -55,7 +58,7 @@ def attend(query, key, value, position, scale, config=None):
     return out
 
 
-#: Head dimension and query heads per KV head the fused RoPE prologue takes (the QUAD kind).
+#: Head dimension and query heads per KV head the fused RoPE prologue takes (the QUAD kind, on either of its kernels).
 ROPE_DIM, ROPE_MAX_GROUP = 128, 4
 
 
