@@ -218,24 +218,21 @@ __global__ __launch_bounds__(512) void flow_kernel(ProjArgs a, int tiles) {
   for (int f = 0; f < OV; ++f)
     if (wf < F) issue_w();
 
-  // A ragged last segment: nothing past K, for the norm's sums and, as the gain read there may be infinite,
-  // once more after it.
+  // A ragged last segment: nothing past K. Its gain, which may be infinite, is cleared in LDS (it came before
+  // x), since operands cleared once more after the norm take 0.5 to 1 % of a launch at up to 8 rows.
   const int tail = (K & 127) && (segs - 1) % KW == kw ? (segs - 1) / KW : -1;  // its unit, or -1
-  auto clear_tail = [&]() {
-    unroll_for<0, CM>([&](auto J) {
-      constexpr int j = decltype(J)::value;
-      if (j == tail) {
-        const u32x4_t zero = {0u, 0u, 0u, 0u};
+  unroll_for<0, CM>([&](auto J) {
+    constexpr int j = decltype(J)::value;
+    if (j == tail) {
+      const u32x4_t zero = {0u, 0u, 0u, 0u};
 #pragma unroll
-        for (int s = 0; s < 4; ++s)
-          if ((j * KW + kw) * 128 + 32 * s + 8 * g >= K) {
+      for (int s = 0; s < 4; ++s)
+        if ((j * KW + kw) * 128 + 32 * s + 8 * g >= K) {
 #pragma unroll
-            for (int m = 0; m < MB; ++m) xr[j][m][s] = zero;
-          }
-      }
-    });
-  };
-  clear_tail();
+          for (int m = 0; m < MB; ++m) xr[j][m][s] = zero;
+        }
+    }
+  });
 
   // ---- RMSNorm: the rows' sums of squares from the operands, then the operands normalised in place
   if constexpr (PRO) {
@@ -250,6 +247,11 @@ __global__ __launch_bounds__(512) void flow_kernel(ProjArgs a, int tiles) {
       ss += __shfl_xor(ss, 16);
       ss += __shfl_xor(ss, 32);
       if (g == 0) ds_put(red_at + 4 * (kw * 16 * MB + 16 * m + li), ss);
+    }
+    if (tail >= 0 && g == 0 && (tail * KW + kw) * 128 + 8 * li >= K) {
+      const uint32_t to = lds_address(gain) + 16 * (kw * GS + 16 * tail + li);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) ds_put(to + 4 * i, 0.f);
     }
     lds_barrier();
     float scale[MB];
@@ -269,7 +271,6 @@ __global__ __launch_bounds__(512) void flow_kernel(ProjArgs a, int tiles) {
 #pragma unroll
         for (int s = 0; s < 4; ++s) xr[j][m][s] = norm8(xr[j][m][s], gn[s], scale[m]);
     });
-    clear_tail();
   }
 
   // ---- epilogue of the parked tiles done .. done + count - 1: thread e takes (tile, column block, lane position);
