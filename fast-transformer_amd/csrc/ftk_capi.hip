@@ -325,8 +325,8 @@ static bool tiles_first(int64_t M, int64_t N, int64_t K, int cus, bool stage, bo
 // Every other projection: FLOW, whose workgroups each load, sum and normalise x before their first product,
 // so it needs tiles enough for that.
 //   5..8 rows beside QUAD (the norm, STORE): more tiles than half the CUs (at 5 rows 2048 x 2048 5.3 / 6.2,
-//     12288 x 2048 13.7 / 11.5, 3072 x 1024 5.1 / 4.9), at up to 6 rows and K past 1024 more tiles than CUs
-//     (4096 x 3072 8.9 / 9.3).
+//     12288 x 2048 13.7 / 11.5, 3072 x 1024 5.1 / 4.9), at up to 6 rows and K past 1024 not from 5/8 of the CUs
+//     to all (4096 x 3072 8.9 / 9.3; 2560 x 3072, in its layer 8.03 / 7.90).
 //   2..4 rows beside QUAD: gate/up from 1.5 tiles per CU and 1024 of K (4 rows 6144 x 1024 6.1 / 5.9, 4096 x
 //     2048 6.7 / 7.3, 12288 x 2048 12.6 / 12.1, 6144 x 3072 10.9 / 11.0), at K = 1024 to 6 per CU (24576 x
 //     1024 13.3 / 12.5, 27648 13.8 / 14.7), without the norm past half the CUs (3 rows 2048 x 3072 5.2 / 5.5,
@@ -335,8 +335,10 @@ static bool tiles_first(int64_t M, int64_t N, int64_t K, int cus, bool stage, bo
 //     RING is built for (4096) QUAD stays: with the norm FLOW is 0.74 to 1.03 times as fast.
 //   2..4 rows beside GEMV: nearly everywhere (19456 x 2560 at 2 / 4 rows 23.8 / 21.0, 34.5 / 20.9; norm 2048 x
 //     2560 at 4 rows 9.9 / 7.4). Not the few tiles of a GEMV whose waves split K (norm, 1024 x 5120 at 2 / 3
-//     rows 7.2 / 10.1, 9.3 / 10.2), nor with the norm two ranges of K at two rows: 1024..2048 with one to 2.5
-//     tiles per CU (gate/up 6144 x 1600 7.9 / 8.4) and 3072..4096 with at most one (4096 x 3584 10.6 / 11.4).
+//     rows 7.2 / 10.1, 9.3 / 10.2; on that line itself gate/up, except with the norm at 2 and 3 rows, is FLOW's:
+//     512 x 5120 without it at 4 rows 6.4 / 6.0). Nor, with the norm at two rows, two ranges of K: 1024..2048 with
+//     one to 2.5 tiles per CU (gate/up 6144 x 1600 7.9 / 8.4; from two where only one wave has a second segment,
+//     8192 x 1152 7.6 / 7.3) and 3072..4096 with at most one (4096 x 3584 10.6 / 11.4).
 //   One row, where only GEMV is built: from more than two tiles per CU (norm 8192 x 2560 10.4 / 11.4, 9216
 //     14.7 / 12.4; gate/up 9216 x 2560 14.5 / 12.9, 19456 23.4 / 20.8).
 static bool flow_first(int64_t M, int epi, bool pro, int64_t N, int64_t K, int cus, bool quad, bool stage, bool stream) {
@@ -344,7 +346,7 @@ static bool flow_first(int64_t M, int epi, bool pro, int64_t N, int64_t K, int c
   const int64_t tiles = flow_tiles(epi, (int)N, kFlowTile);
   if (M > 4) {
     if (stage) return false;
-    return !quad || tiles > (M <= 6 && K > 1024 ? cus : cus / 2);
+    return !quad || (tiles > cus / 2 && (M > 6 || K <= 1024 || tiles > cus || 8 * tiles <= 5ll * cus));
   }
   if (M == 1) return !stream && tiles > 2ll * cus;
   if (quad) {
@@ -355,9 +357,12 @@ static bool flow_first(int64_t M, int epi, bool pro, int64_t N, int64_t K, int c
   }
   if (stream) return false;
   if (epi == FTK_EPI_ARGMAX) return true;
-  if (gemv_default(epi, N, K).kw > 1) return tiles > (epi == FTK_EPI_SWIGLU && pro ? 2 * cus : cus) >> (M - 1);
+  if (gemv_default(epi, N, K).kw > 1) {
+    const int64_t few = (epi == FTK_EPI_SWIGLU && pro ? 2 * cus : cus) >> (M - 1);
+    return tiles > few || (tiles == few && epi == FTK_EPI_SWIGLU && (!pro || M == 4));
+  }
   if (M > 2 || !pro) return true;
-  if (K > 1024 && K < 2048) return tiles <= cus || 2 * tiles > 5ll * cus;
+  if (K > 1024 && K < 2048) return tiles <= (K <= 1152 ? 2ll : 1ll) * cus || 2 * tiles > 5ll * cus;
   return !(K > 3072 && K < 4096 && tiles <= cus);
 }
 

@@ -17,6 +17,7 @@ LINES = [
     (5, 1024, 2048, STORE, True, QUAD), (5, 2048, 2048, STORE, True, QUAD), (8, 2048, 3072, STORE, True, QUAD),
     (6, 4096, 3072, STORE, True, QUAD), (8, 4096, 3072, STORE, True, FLOW), (5, 4096, 1024, STORE, True, FLOW),
     (5, 6144, 2048, STORE, True, FLOW), (8, 1024, 1024, STORE, True, QUAD), (9, 1024, 2048, STORE, True, FLOW),
+    (5, 2560, 3072, STORE, True, FLOW), (5, 2576, 3072, STORE, True, QUAD), (6, 4112, 3072, STORE, True, FLOW),
     # gate/up beside QUAD, 3..4 rows
     (3, 2048, 2048, SWIGLU, True, QUAD), (4, 6144, 3072, SWIGLU, True, QUAD), (4, 6144, 1024, SWIGLU, True, FLOW),
     (3, 12288, 2048, SWIGLU, True, FLOW), (4, 24576, 1024, SWIGLU, True, FLOW), (4, 27648, 1024, SWIGLU, True, QUAD),
@@ -28,6 +29,9 @@ LINES = [
     (2, 4096, 5120, SWIGLU, True, GEMV), (2, 6144, 5120, SWIGLU, True, FLOW), (2, 4096, 3584, STORE, True, GEMV),
     (2, 6144, 3584, STORE, True, FLOW), (2, 10240, 1280, SWIGLU, True, GEMV), (2, 12288, 1280, SWIGLU, True, FLOW),
     (3, 10240, 1280, SWIGLU, True, FLOW), (2, 10240, 1280, SWIGLU, False, FLOW), (4, 1024, 5120, STORE, True, FLOW),
+    (4, 512, 5120, SWIGLU, False, FLOW), (4, 496, 5120, SWIGLU, False, GEMV), (4, 1024, 5120, SWIGLU, True, FLOW),
+    (3, 2048, 5120, SWIGLU, True, GEMV), (2, 8192, 1152, STORE, True, FLOW), (2, 8208, 1152, STORE, True, GEMV),
+    (2, 8192, 1160, STORE, True, GEMV),
     # beside GEMV, one row
     (1, 8192, 2560, STORE, True, GEMV), (1, 9216, 2560, STORE, True, FLOW), (1, 9216, 2560, SWIGLU, True, FLOW),
     # plain projections
